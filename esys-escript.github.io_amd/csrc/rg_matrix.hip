@@ -156,149 +156,329 @@ __device__ __forceinline__ const double* coef_pt(const CoefDev& c, int64_t e, in
     return (c.mode == RG_COEF_EXPANDED) ? p + q * dps : p;
 }
 
+// Nodes whose (k, m) pairs one wave holds.
+template <int NB>
+__host__ __device__ constexpr int asm_nodes_per_wave()
+{
+    return 64 / (NB * NB);
+}
+
 // Colour-free gather assembly.  One thread per (node i, equation k,
-// component m): it visits the 2^DIM elements around node i, computes row a
-// (the node's local index) of each element matrix by Gauss quadrature and
-// adds entry (a, b) to the stencil slot of local node b:
-//   EM_S[k,m,a,b] = sum_q w ( A[k,i,m,j] dN_a/dx_i dN_b/dx_j + B[k,i,m] N_b dN_a/dx_i
-//                           + C[k,m,j] N_a dN_b/dx_j + D[k,m] N_a N_b )
-//   EM_F[k,a]     = sum_q w ( X[k,i] dN_a/dx_i + Y[k] N_a )
+// component m): it visits the 2^DIM elements around node i, forms row a (the
+// node's local index) of each element matrix and adds entry (a, b) to the
+// stencil slot of local node b:
+//   EM_S[k,m,a,b] = int A[k,i,m,j] dN_a/dx_i dN_b/dx_j + B[k,i,m] N_b dN_a/dx_i
+//                     + C[k,m,j] N_a dN_b/dx_j + D[k,m] N_a N_b
+//   EM_F[k,a]     = int X[k,i] dN_a/dx_i + Y[k] N_a
 // -- the weak form that DefaultAssembler3D::assemblePDESingle/System
-// integrate with the same 2-point Gauss rule (points (1-+1/sqrt3)/2, x
-// fastest; ripley/src/DefaultAssembler3D.cpp:153-2229, :3631-5745) and, for
-// reduced, the one-point rule of assemblePDE*Reduced (:2891-3270).  Each
-// matrix entry and rhs entry is written by exactly one thread: no atomics.
+// integrate with the 2-point Gauss rule (points (1-+1/sqrt3)/2, x fastest;
+// ripley/src/DefaultAssembler3D.cpp:153-2229, :3631-5745) and, for reduced,
+// the one-point rule of assemblePDE*Reduced (:2891-3270).  Each matrix entry
+// and rhs entry is written by exactly one thread: no atomics.
+//
+// Coefficients with one point per element (GAUSS = false) are integrated in
+// closed form (the 2-point rule is exact for these products): along an axis
+// int N N = 1/3 or 1/6 for equal / different local coordinates, int N' N =
+// +-1/2, int N' N' = +-1 in units of h, so an entry takes one multiply-add
+// per coefficient component instead of one Gauss sum.  Coefficients on
+// quadrature points and the one-point rule (GAUSS = true) take the Gauss sum,
+// the point loop outermost so that the shape functions of a point serve all
+// elements.  Both in one kernel took 256 registers (one wave per SIMD); a PDE
+// with both kinds runs one launch of each.
+//
+// Bound: the coefficient reads.  A data point of a system is NB^2 DIM^2 (A)
+// contiguous doubles of which thread (k, m) needs every NB-th, so the lanes
+// of a wave are the NB^2 pairs (k, m) of 64 / NB^2 neighbouring nodes: one
+// load instruction then covers whole runs of a data point, and the block's
+// four waves take 2 x 2 neighbouring node lines (3-D; four lines in 2-D),
+// which share their elements through L1.  With one (k, m) per blockIdx.y and
+// lanes along x, each load touched 64 lines: Brick 48x47x49, 3 equations,
+// A per element and the rest on quadrature points 10.48 ms -> 0.17 + 1.09 ms (bytes alone 0.24 ms);
+// Brick 96^3 elasticity (A per element, symmetric storage) 37.6 -> 0.92 ms (bytes alone 0.30 ms).
+template <int DIM, int NB>
+struct AsmNode {
+    int k, m;            // equation and component of the thread
+    int64_t x, y, z, i;  // its node
+    bool valid;
+    int64_t e0;          // element at (x - 1, y - 1, z - 1)
+    unsigned in;         // bit t: element t = (ex, ey, ez) at node index - 1 + t is in the grid
+    __device__ __forceinline__ AsmNode(const AsmArgs& a, int64_t tiles_x, int64_t tiles_y)
+    {
+        constexpr int PAIRS = NB * NB, NPW = asm_nodes_per_wave<NB>();
+        const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+        const int km = lane % PAIRS;
+        k = km % NB;
+        m = km / NB;
+        const int64_t bx = blockIdx.x % tiles_x, by = (blockIdx.x / tiles_x) % tiles_y,
+                      bz = blockIdx.x / (tiles_x * tiles_y);
+        x = bx * NPW + lane / PAIRS;
+        y = (DIM == 3) ? by * 2 + (wv & 1) : by * 4 + wv;
+        z = (DIM == 3) ? bz * 2 + (wv >> 1) : 0;
+        valid = lane < PAIRS * NPW && x < a.n0 && y < a.n1 && (DIM == 2 || z < a.n2);
+        i = x + a.n0 * (y + (DIM == 3 ? a.n1 * z : 0));
+        e0 = (x - 1) + (int64_t)a.ne0 * ((y - 1) + (DIM == 3 ? (int64_t)a.ne1 * (z - 1) : 0));
+        in = 0;
+#pragma unroll
+        for (int t = 0; t < (1 << DIM); ++t) {
+            const int64_t k0 = x - 1 + (t & 1), k1 = y - 1 + ((t >> 1) & 1), k2 = (DIM == 3) ? z - 1 + (t >> 2) : 0;
+            if (k0 >= 0 && k0 < a.ne0 && k1 >= 0 && k1 < a.ne1 && (DIM == 2 || (k2 >= 0 && k2 < a.ne2))) in |= 1u << t;
+        }
+    }
+    __device__ __forceinline__ int64_t element(const AsmArgs& a, int t) const
+    {
+        return e0 + (t & 1) + (int64_t)a.ne0 * (((t >> 1) & 1) + (DIM == 3 ? (int64_t)a.ne1 * (t >> 2) : 0));
+    }
+};
+
+// Stencil slot of local node b of element t, seen from the node.
+template <int DIM>
+__host__ __device__ constexpr int asm_slot(int t, int b)
+{
+    return ((t & 1) + (b & 1)) + 3 * (((t >> 1) & 1) + ((b >> 1) & 1)) + (DIM == 3 ? 9 * ((t >> 2) + (b >> 2)) : 0);
+}
+
 template <int DIM, int NB, bool SYM>
-__global__ __launch_bounds__(kBlock) void k_assemble(AsmArgs a, double* __restrict__ val, int64_t ld,
-                                                     int64_t N, double* __restrict__ rhs)
+__device__ __forceinline__ void asm_store(const AsmNode<DIM, NB>& nd, const double (&acc)[StencilShape<DIM>::NS],
+                                          double* __restrict__ val, int64_t ld, bool zero)
+{
+    constexpr int FIRST = SYM ? StencilShape<DIM>::CENTER : 0;
+#pragma unroll
+    for (int t = 0; t < stored_slots<DIM, SYM>(); ++t) {
+        double* p = &val[(int64_t)(t * NB * NB + nd.k + NB * nd.m) * ld + nd.i];
+        if (zero) *p = acc[FIRST + t];
+        else *p += acc[FIRST + t];
+    }
+}
+
+template <int DIM, int NB, bool SYM>
+__global__ __launch_bounds__(kBlock) void k_assemble_const(AsmArgs a, double* __restrict__ val, int64_t ld,
+                                                           int64_t tiles_x, int64_t tiles_y, bool zero,
+                                                           double* __restrict__ rhs)
 {
     constexpr int NS = StencilShape<DIM>::NS;
-    constexpr int CEN = StencilShape<DIM>::CENTER;
-    constexpr int NST = stored_slots<DIM, SYM>();
-    constexpr int FIRST = SYM ? CEN : 0;
     constexpr int NNODE = 1 << DIM;
-    const int km = blockIdx.y;
-    const int k = km % NB, m = km / NB;
-    const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-    if (i >= N) return;
-    const int64_t x = i % a.n0, y = (i / a.n0) % a.n1, z = (DIM == 3) ? i / (a.n0 * a.n1) : 0;
-    const double h[3] = {a.h0, a.h1, a.h2};
+    const AsmNode<DIM, NB> nd(a, tiles_x, tiles_y);
+    if (!nd.valid) return;
+    const int k = nd.k, m = nd.m;
+    const double ih[3] = {1.0 / a.h0, 1.0 / a.h1, 1.0 / a.h2};
     double vol = a.h0 * a.h1;
     if (DIM == 3) vol *= a.h2;
-    const int nq = a.reduced ? 1 : NNODE;
-    const double w = vol / nq;
-    const double g0 = 0.5 - 0.5 / 1.73205080756887719318, g1 = 0.5 + 0.5 / 1.73205080756887719318;
     const bool doS = (a.A.mode | a.B.mode | a.C.mode | a.D.mode) != 0;
     const bool doF = rhs != nullptr && m == 0 && (a.X.mode | a.Y.mode) != 0;
-    const int dpsA = NB * DIM * NB * DIM, dpsB = NB * DIM * NB, dpsC = NB * NB * DIM, dpsD = NB * NB;
-    const int dpsX = NB * DIM, dpsY = NB;
-
     double acc[NS];
 #pragma unroll
     for (int s = 0; s < NS; ++s) acc[s] = 0.0;
     double f = 0.0;
-
 #pragma unroll
-    for (int ez = 0; ez < (DIM == 3 ? 2 : 1); ++ez)
+    for (int t = 0; t < NNODE; ++t) {
+        if (nd.in & (1u << t)) {
+            const int64_t e = nd.element(a, t);
+            double A[DIM][DIM], B[DIM], C[DIM], D = 0.0;
 #pragma unroll
-        for (int ey = 0; ey < 2; ++ey)
+            for (int p = 0; p < DIM; ++p) {
+                B[p] = C[p] = 0.0;
 #pragma unroll
-            for (int ex = 0; ex < 2; ++ex) {
-                const int64_t k0 = x - 1 + ex, k1 = y - 1 + ey, k2 = (DIM == 3) ? z - 1 + ez : 0;
-                if (k0 < 0 || k0 >= a.ne0 || k1 < 0 || k1 >= a.ne1) continue;
-                if (DIM == 3 && (k2 < 0 || k2 >= a.ne2)) continue;
-                const int64_t e = k0 + (int64_t)a.ne0 * (k1 + (int64_t)a.ne1 * k2);
-                // local index bits of node i in this element
-                const int abit[3] = {1 - ex, 1 - ey, 1 - ez};
-                for (int q = 0; q < nq; ++q) {
-                    double xi[3];
+                for (int j = 0; j < DIM; ++j) A[p][j] = 0.0;
+            }
+            if (a.A.mode) {
+                const double* P = a.A.p + (int64_t)a.A.stride * e;
+                if (a.A.iso) {
 #pragma unroll
-                    for (int d = 0; d < DIM; ++d) xi[d] = a.reduced ? 0.5 : (((q >> d) & 1) ? g1 : g0);
-                    double fa[3], Ga[3];
+                    for (int p = 0; p < DIM; ++p) A[p][p] = P[0] * (vol * ih[p] * ih[p]);
+                } else {
 #pragma unroll
-                    for (int d = 0; d < DIM; ++d) fa[d] = abit[d] ? xi[d] : 1.0 - xi[d];
-                    double Na = fa[0] * fa[1];
-                    if (DIM == 3) Na *= fa[2];
+                    for (int j = 0; j < DIM; ++j)
 #pragma unroll
-                    for (int d = 0; d < DIM; ++d) {
-                        double gq = (abit[d] ? 1.0 : -1.0) / h[d];
-#pragma unroll
-                        for (int o = 0; o < DIM; ++o)
-                            if (o != d) gq *= fa[o];
-                        Ga[d] = gq;
-                    }
-                    if (doS) {
-                        double u[3] = {0.0, 0.0, 0.0};
-                        double c0 = 0.0;
-                        if (a.A.mode) {
-                            const double* Ap = coef_pt(a.A, e, q, a.A.iso ? 1 : dpsA);
-                            if (a.A.iso) {
-#pragma unroll
-                                for (int j = 0; j < DIM; ++j) u[j] = Ap[0] * Ga[j];
-                            } else {
-#pragma unroll
-                                for (int j = 0; j < DIM; ++j)
-#pragma unroll
-                                    for (int ii = 0; ii < DIM; ++ii)
-                                        u[j] += Ap[k + NB * (ii + DIM * (m + NB * j))] * Ga[ii];
-                            }
-                        }
-                        if (a.C.mode) {
-                            const double* Cp = coef_pt(a.C, e, q, dpsC);
-#pragma unroll
-                            for (int j = 0; j < DIM; ++j) u[j] += Na * Cp[k + NB * (m + NB * j)];
-                        }
-                        if (a.B.mode) {
-                            const double* Bp = coef_pt(a.B, e, q, dpsB);
-#pragma unroll
-                            for (int ii = 0; ii < DIM; ++ii) c0 += Bp[k + NB * (ii + DIM * m)] * Ga[ii];
-                        }
-                        if (a.D.mode) {
-                            const double* Dp = coef_pt(a.D, e, q, dpsD);
-                            c0 += Dp[k + NB * m] * Na;
-                        }
-#pragma unroll
-                        for (int b = 0; b < NNODE; ++b) {
-                            const int bb[3] = {b & 1, (b >> 1) & 1, (b >> 2) & 1};
-                            double fb[3];
-#pragma unroll
-                            for (int d = 0; d < DIM; ++d) fb[d] = bb[d] ? xi[d] : 1.0 - xi[d];
-                            double Nb = fb[0] * fb[1];
-                            if (DIM == 3) Nb *= fb[2];
-                            double sdot = c0 * Nb;
-#pragma unroll
-                            for (int d = 0; d < DIM; ++d) {
-                                double gq = (bb[d] ? 1.0 : -1.0) / h[d];
-#pragma unroll
-                                for (int o = 0; o < DIM; ++o)
-                                    if (o != d) gq *= fb[o];
-                                sdot += u[d] * gq;
-                            }
-                            const int s = (ex + bb[0]) + 3 * (ey + bb[1]) + (DIM == 3 ? 9 * (ez + bb[2]) : 0);
-                            acc[s] += w * sdot;
-                        }
-                    }
-                    if (doF) {
-                        double sf = 0.0;
-                        if (a.X.mode) {
-                            const double* Xp = coef_pt(a.X, e, q, dpsX);
-#pragma unroll
-                            for (int ii = 0; ii < DIM; ++ii) sf += Xp[k + NB * ii] * Ga[ii];
-                        }
-                        if (a.Y.mode) {
-                            const double* Yp = coef_pt(a.Y, e, q, dpsY);
-                            sf += Yp[k] * Na;
-                        }
-                        f += w * sf;
-                    }
+                        for (int p = 0; p < DIM; ++p)
+                            A[p][j] = P[k + NB * (p + DIM * (m + NB * j))] * (vol * ih[p] * ih[j]);
                 }
             }
+            if (a.B.mode) {
+                const double* P = a.B.p + (int64_t)a.B.stride * e;
+#pragma unroll
+                for (int p = 0; p < DIM; ++p) B[p] = P[k + NB * (p + DIM * m)] * (vol * ih[p]);
+            }
+            if (a.C.mode) {
+                const double* P = a.C.p + (int64_t)a.C.stride * e;
+#pragma unroll
+                for (int p = 0; p < DIM; ++p) C[p] = P[k + NB * (m + NB * p)] * (vol * ih[p]);
+            }
+            if (a.D.mode) D = (a.D.p + (int64_t)a.D.stride * e)[k + NB * m] * vol;
+#pragma unroll
+            for (int b = 0; b < NNODE; ++b) {
+                const int s = asm_slot<DIM>(t, b);
+                if (SYM && s < StencilShape<DIM>::CENTER) continue;
+                // signs of dN_a, dN_b and int N_a N_b / h along each axis
+                double sa[DIM], sb[DIM], mass[DIM];
+#pragma unroll
+                for (int p = 0; p < DIM; ++p) {
+                    const int ab = 1 - ((t >> p) & 1), bb = (b >> p) & 1;
+                    sa[p] = ab ? 1.0 : -1.0;
+                    sb[p] = bb ? 1.0 : -1.0;
+                    mass[p] = ab == bb ? 1.0 / 3.0 : 1.0 / 6.0;
+                }
+                double full = 1.0, r = acc[s];
+#pragma unroll
+                for (int p = 0; p < DIM; ++p) full *= mass[p];
+#pragma unroll
+                for (int p = 0; p < DIM; ++p)
+#pragma unroll
+                    for (int j = 0; j < DIM; ++j) {
+                        double c = (p == j) ? sa[p] * sb[p] : 0.25 * sa[p] * sb[j];
+#pragma unroll
+                        for (int o = 0; o < DIM; ++o)
+                            if (o != p && o != j) c *= mass[o];
+                        r = fma(A[p][j], c, r);
+                    }
+                if (a.B.mode | a.C.mode) {
+#pragma unroll
+                    for (int p = 0; p < DIM; ++p) {
+                        double c = 0.5;
+#pragma unroll
+                        for (int o = 0; o < DIM; ++o)
+                            if (o != p) c *= mass[o];
+                        r = fma(B[p], c * sa[p], r);
+                        r = fma(C[p], c * sb[p], r);
+                    }
+                }
+                acc[s] = fma(D, full, r);
+            }
+            if (doF) {
+                if (a.X.mode) {
+                    const double* P = a.X.p + (int64_t)a.X.stride * e;
+#pragma unroll
+                    for (int p = 0; p < DIM; ++p) {
+                        const double c = ((t >> p) & 1) ? -2.0 / NNODE : 2.0 / NNODE;
+                        f = fma(P[k + NB * p], c * (vol * ih[p]), f);
+                    }
+                }
+                if (a.Y.mode) f = fma((a.Y.p + (int64_t)a.Y.stride * e)[k], vol * (1.0 / NNODE), f);
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);   // the next element's loads stay behind: half the registers
+    }
+    if (doS) asm_store<DIM, NB, SYM>(nd, acc, val, ld, zero);
+    if (doF) rhs[nd.i * NB + k] += f;
+}
+
+template <int DIM, int NB, bool SYM>
+__global__ __launch_bounds__(kBlock) void k_assemble_gauss(AsmArgs a, double* __restrict__ val, int64_t ld,
+                                                           int64_t tiles_x, int64_t tiles_y, bool zero,
+                                                           double* __restrict__ rhs)
+{
+    constexpr int NS = StencilShape<DIM>::NS;
+    constexpr int NNODE = 1 << DIM;
+    const AsmNode<DIM, NB> nd(a, tiles_x, tiles_y);
+    if (!nd.valid) return;
+    const int k = nd.k, m = nd.m;
+    const double ih[3] = {1.0 / a.h0, 1.0 / a.h1, 1.0 / a.h2};
+    double vol = a.h0 * a.h1;
+    if (DIM == 3) vol *= a.h2;
+    const bool doS = (a.A.mode | a.B.mode | a.C.mode | a.D.mode) != 0;
+    const bool doF = rhs != nullptr && m == 0 && (a.X.mode | a.Y.mode) != 0;
+    constexpr int dpsA = NB * DIM * NB * DIM, dpsB = NB * DIM * NB, dpsC = NB * NB * DIM, dpsD = NB * NB;
+    constexpr int dpsX = NB * DIM, dpsY = NB;
+    double acc[NS];
+#pragma unroll
+    for (int s = 0; s < NS; ++s) acc[s] = 0.0;
+    double f = 0.0;
+    const int nq = a.reduced ? 1 : NNODE;
+    const double w = vol / nq;
+    const double g0 = 0.5 - 0.5 / 1.73205080756887719318, g1 = 0.5 + 0.5 / 1.73205080756887719318;
+#pragma unroll 1
+    for (int q = 0; q < nq; ++q) {
+        double phi[DIM][2];   // 1-D shape functions at the point
+#pragma unroll
+        for (int p = 0; p < DIM; ++p) {
+            phi[p][1] = a.reduced ? 0.5 : (((q >> p) & 1) ? g1 : g0);
+            phi[p][0] = 1.0 - phi[p][1];
+        }
+        // N[b], and |dN_b/dx_p| by the bits of b along the other axes (its
+        // sign is a compile-time one at each use)
+        double N[NNODE], M[DIM][NNODE / 2];
+#pragma unroll
+        for (int b = 0; b < NNODE; ++b) {
+            N[b] = 1.0;
+#pragma unroll
+            for (int p = 0; p < DIM; ++p) N[b] *= phi[p][(b >> p) & 1];
+        }
+#pragma unroll
+        for (int p = 0; p < DIM; ++p)
+#pragma unroll
+            for (int r = 0; r < NNODE / 2; ++r) {
+                const int o1 = p == 0 ? 1 : 0, o2 = p == 2 ? 1 : 2;
+                M[p][r] = ih[p] * phi[o1][r & 1];
+                if (DIM == 3) M[p][r] *= phi[DIM == 3 ? o2 : 0][r >> 1];
+            }
+        auto G = [&](int b, int p) {
+            const int b1 = (b >> (p == 0 ? 1 : 0)) & 1, b2 = DIM == 3 ? (b >> (p == 2 ? 1 : 2)) & 1 : 0;
+            const double g = M[p][b1 + 2 * b2];
+            return ((b >> p) & 1) ? g : -g;
+        };
+#pragma unroll
+        for (int t = 0; t < NNODE; ++t) {
+            if (nd.in & (1u << t)) {
+                // opaque per use: the addresses of all elements' points, kept
+                // over the point loop, took 100 registers
+                int64_t e = nd.element(a, t);
+                asm volatile("" : "+v"(e));
+                const int la = (NNODE - 1) - t;   // the node's local index in element t
+                double u[DIM], c0 = 0.0;
+#pragma unroll
+                for (int j = 0; j < DIM; ++j) u[j] = 0.0;
+                if (a.A.mode) {
+                    const double* P = coef_pt(a.A, e, q, a.A.iso ? 1 : dpsA);
+                    if (a.A.iso) {
+#pragma unroll
+                        for (int j = 0; j < DIM; ++j) u[j] = P[0] * G(la, j);
+                    } else {
+#pragma unroll
+                        for (int j = 0; j < DIM; ++j)
+#pragma unroll
+                            for (int p = 0; p < DIM; ++p)
+                                u[j] = fma(P[k + NB * (p + DIM * (m + NB * j))], G(la, p), u[j]);
+                    }
+                }
+                if (a.C.mode) {
+                    const double* P = coef_pt(a.C, e, q, dpsC);
+#pragma unroll
+                    for (int j = 0; j < DIM; ++j) u[j] = fma(P[k + NB * (m + NB * j)], N[la], u[j]);
+                }
+                if (a.B.mode) {
+                    const double* P = coef_pt(a.B, e, q, dpsB);
+#pragma unroll
+                    for (int p = 0; p < DIM; ++p) c0 = fma(P[k + NB * (p + DIM * m)], G(la, p), c0);
+                }
+                if (a.D.mode) c0 = fma(coef_pt(a.D, e, q, dpsD)[k + NB * m], N[la], c0);
+                if (doS) {
+#pragma unroll
+                    for (int b = 0; b < NNODE; ++b) {
+                        const int s = asm_slot<DIM>(t, b);
+                        if (SYM && s < StencilShape<DIM>::CENTER) continue;
+                        double r = fma(c0, N[b], acc[s]);
+#pragma unroll
+                        for (int j = 0; j < DIM; ++j) r = fma(u[j], G(b, j), r);
+                        acc[s] = r;
+                    }
+                }
+                if (doF) {
+                    if (a.X.mode) {
+                        const double* P = coef_pt(a.X, e, q, dpsX);
+#pragma unroll
+                        for (int p = 0; p < DIM; ++p) f = fma(P[k + NB * p], G(la, p), f);
+                    }
+                    if (a.Y.mode) f = fma(coef_pt(a.Y, e, q, dpsY)[k], N[la], f);
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
     if (doS) {
 #pragma unroll
-        for (int t = 0; t < NST; ++t)
-            val[(int64_t)(t * NB * NB + k + NB * m) * ld + i] += acc[FIRST + t];
+        for (int s = 0; s < NS; ++s) acc[s] *= w;
+        asm_store<DIM, NB, SYM>(nd, acc, val, ld, zero);
     }
-    if (doF) rhs[i * NB + k] += f;
+    if (doF) rhs[nd.i * NB + k] += w * f;
 }
 
 // Element-constant isotropic A = kappa_e I (single PDE, full quadrature),
@@ -613,10 +793,34 @@ void launch_assemble(rg_matrix* m, const rg_pde_coefs& c, int reduced, double* r
             else byz(IC<2>{}, BC<false>{});
         }
     } else {
-        const dim3 grid((unsigned)((g.N + kBlock - 1) / kBlock), (unsigned)(g.bs * g.bs));
+        // the coefficients of each kernel (k_assemble_const, k_assemble_gauss)
+        AsmArgs ac = a, ag = a;
+        CoefDev* const both[6][2] = {{&ac.A, &ag.A}, {&ac.B, &ag.B}, {&ac.C, &ag.C},
+                                     {&ac.D, &ag.D}, {&ac.X, &ag.X}, {&ac.Y, &ag.Y}};
+        bool is_const = false, is_gauss = false;
+        for (auto& p : both) {
+            const int mode = p[0]->mode;
+            const bool cst = !reduced && mode == RG_COEF_ELEMENT;
+            is_const = is_const || cst;
+            is_gauss = is_gauss || (mode && !cst);
+            p[cst ? 1 : 0]->mode = RG_COEF_EMPTY;
+        }
         dispatch(g, m->symmetric, [&](auto D, auto B, auto S) {
-            hipLaunchKernelGGL((k_assemble<D.value, B.value, S.value>), grid, dim3(kBlock), 0,
-                               m->ctx->stream, a, m->val, g.ld, g.N, rhs);
+            constexpr int npw = asm_nodes_per_wave<B.value>();
+            const int64_t ly = D.value == 3 ? 2 : 4;   // node lines per block along y (and 2 along z in 3-D)
+            const int64_t tx = (g.nn[0] + npw - 1) / npw, ty = (g.nn[1] + ly - 1) / ly,
+                          tz = D.value == 3 ? (g.nn[2] + 1) / 2 : 1;
+            RG_CHECK(tx * ty * tz < ((int64_t)1 << 31), RG_VALUE_ERROR, "assemble: grid too large");
+            const dim3 grid((unsigned)(tx * ty * tz));
+            bool zero = m->val_zero;
+            if (is_const) {
+                hipLaunchKernelGGL((k_assemble_const<D.value, B.value, S.value>), grid, dim3(kBlock), 0, m->ctx->stream,
+                                   ac, m->val, g.ld, tx, ty, zero, rhs);
+                if (ac.A.mode || ac.B.mode || ac.C.mode || ac.D.mode) zero = false;
+            }
+            if (is_gauss)
+                hipLaunchKernelGGL((k_assemble_gauss<D.value, B.value, S.value>), grid, dim3(kBlock), 0, m->ctx->stream,
+                                   ag, m->val, g.ld, tx, ty, zero, rhs);
         });
     }
     RG_HIP(hipGetLastError());
