@@ -92,7 +92,9 @@ struct KrylovState {
     // coefficients of the w recurrence, c * eta for the x update and the
     // scaling of the preconditioned residual norm
     double c, c_old, s, s_old, a1, a2, a3, ceta, norm_scal;
-    double pend_rz, pend_rr, pad2;
+    double pend_rz, pend_rr;
+    int32_t gave_up;        // one-launch solve: a workgroup stopped waiting for the others
+    int32_t pad2;
 };
 enum { KS_RUNNING = 0, KS_CONVERGED = 1, KS_MAXITER = 2, KS_BREAKDOWN = 3, KS_STAGNATED = 4, KS_NEGATIVE = 5 };
 
@@ -123,6 +125,9 @@ struct rg_solver_work {
     double* norms = nullptr;        // [0] sum of squares, [1] max abs
     rg::KrylovState* st = nullptr;
     int* flag = nullptr;
+    void* slots = nullptr;          // partial sums of the one-launch solve (rg_resident.hip)
+    int res_state[8] = {};          // per method: 0 not looked at, 1 fits in one launch, 2 does not
+    int res_tile[8][3] = {};        // its tile sides
     hipStream_t capture = nullptr;
     hipGraphExec_t graph = nullptr;
     int graph_method = -1, graph_sweeps = -1, graph_iters = -1;

@@ -22,6 +22,7 @@
 #include "rg_dispatch.h"
 #include "rg_krylov.h"
 #include "rg_mg.h"
+#include "rg_resident.h"
 #include "rg_stencil.h"
 
 namespace rg {
@@ -991,6 +992,7 @@ struct SolverImpl {
     Launch L;     // node kernels without pairing (init, Jacobi sweeps)
     int prec = RG_PRECONDITIONER_JACOBI;
     bool nt = false;   // non-temporal vector streams in the update kernels (stream_policy)
+    int polls = 0;     // the caller's check_interval (0: none given)
     const double* norm_w = nullptr;   // the flexible CG's residual norm is taken of r / norm_w
 
     explicit SolverImpl(rg_matrix* mm) : m(mm), w(mm->work), st(mm->ctx->stream), L(chunked_launch(mm->g.N)) {}
@@ -1349,11 +1351,35 @@ struct SolverImpl {
         RG_HIP(hipGraphLaunch(w->graph, st));
     }
 
+    // The Krylov loop in one launch, for systems that fit in the registers
+    // (rg_resident.hip) and one Jacobi sweep; false if it is left to the
+    // launch sequence.  A caller that gives a check_interval gets the launch
+    // sequence, whose host polls it sets.
+    bool one_launch(int method, int sweeps, int maxit, double tol, int* status, int* iters, double* norm)
+    {
+        if (buffered(sweeps)) return false;
+        if (w->res_state[method] == 0) w->res_state[method] = resident_fits(m, method, w->res_tile[method]) ? 1 : 2;
+        if (w->res_state[method] != 1) return false;
+        KrylovState out;
+        if (!resident_solve(m, method, w->res_tile[method], maxit, tol, kResSpins, &out)) {
+            // the iterate may have moved: the launch sequence starts from its residual
+            w->res_state[method] = 2;
+            RG_HIP(hipMemcpyAsync(w->r, w->bb, sizeof(double) * w->n, hipMemcpyDeviceToDevice, st));
+            launch_spmv(m, -1.0, w->xw, 1.0, w->r);
+            return false;
+        }
+        *status = out.status;
+        *iters = out.num_iter;
+        *norm = out.norm;
+        return true;
+    }
+
     // Runs the Krylov loop from w->r, w->xw until the state reports done.
     // Returns (status, iterations, final norm).
     void krylov(int method, int sweeps, int maxit, double tol, int check, bool use_graph, int* status,
                 int* iters, double* norm)
     {
+        if (polls == 0 && one_launch(method, sweeps, maxit, tol, status, iters, norm)) return;
         // the host copy and two polling slots sit below the flag words at pinned + 128
         static_assert(3 * sizeof(KrylovState) <= 128 * sizeof(double), "KrylovState outgrew the pinned buffer");
         KrylovState h;
@@ -1481,6 +1507,7 @@ void ensure_work(rg_matrix* m)
         RG_HIP(hipMalloc(&w->norms, 4 * sizeof(double)));
         RG_HIP(hipMalloc(&w->st, sizeof(KrylovState)));
         RG_HIP(hipMalloc(&w->flag, sizeof(int)));
+        RG_HIP(hipMalloc(&w->slots, resident_slot_bytes()));
     } catch (...) {
         m->work = w;
         throw;
@@ -1498,6 +1525,7 @@ void free_work(rg_solver_work* w)
         if (b) hipFree(b);
     if (w->st) hipFree(w->st);
     if (w->flag) hipFree(w->flag);
+    if (w->slots) hipFree(w->slots);
     delete w;
 }
 
@@ -1576,6 +1604,7 @@ int solve(rg_matrix* m, double* x, const double* b, const rg_options& opt, rg_di
     SolverImpl S(m);
     S.prec = prec;
     S.nt = stream_policy(m, opt.method);
+    S.polls = std::max(0, opt.check_interval);
     const int64_t n = w->n;
     const int vgrid = 2048;
     prepare_solve(m, prec);

@@ -273,7 +273,8 @@ typedef struct {
     int32_t verbose;
     int32_t accept_failed_convergence;
     int32_t check_interval;      /* iterations per replayed graph / host check (0: 32; 1 for
-                                    RG_METHOD_FCG_LEARNED) */
+                                    RG_METHOD_FCG_LEARNED; and systems that fit on the chip
+                                    are solved in one launch without host checks) */
     int32_t criterion;
     int32_t preconditioner;      /* RG_PRECONDITIONER_*, default Jacobi */
 } rg_options;

@@ -1,0 +1,155 @@
+"""The one-launch Krylov solves (systems that fit in the chip's registers) at
+the edges of their tiling, against the oracle's PASO restatement: one tile, a
+few tiles, tiles cut by the grid's end, thin grids, the largest grids that
+still fit and the first that does not; full and symmetric storage.  Bars: the
+oracle's iteration count within 2 % (at least 2), its solution within 1e-6, as
+for every solve; the FP64 residual is checked beside them."""
+import numpy as np
+import pytest
+import torch
+
+import oracle as O
+import ripley_hip as R
+from gpu_helpers import dirichlet_mask, gpu_assemble, grid, to_dev
+
+pytestmark = pytest.mark.gpu
+
+# nodes: 24 and 60 (far fewer than threads), 1-tile sizes, several tiles, and
+# sides that no tile side divides
+SIZES = [(2, (5, 3)), (2, (1, 700)), (2, (44, 43)), (2, (45, 45)), (2, (97, 61)), (2, (200, 131)),
+         (3, (2, 1, 3)), (3, (10, 9, 11)), (3, (11, 11, 11)), (3, (3, 2, 250)), (3, (30, 23, 17))]
+
+
+def _problem(dim, ne, sym, bs=1):
+    rng = np.random.default_rng(sum(ne) + 100 * dim)
+    dom, length = grid(dim, ne)
+    E = dom.getNumElements()
+    A = np.exp(0.7 * rng.standard_normal(E))[:, None, None] * np.eye(dim)[None]
+    Y = rng.uniform(0.5, 1.5, E)
+    op, rhs = gpu_assemble(dom, 1, symmetric=sym, A=A, Y=Y)
+    q = dirichlet_mask(dom, dim - 1)
+    op.nullifyRowsAndCols(to_dev(q), to_dev(q), 1.0)
+    ptr, idx, val, orhs = O.assemble(dim, ne, length, A=A, Y=Y)
+    O.nullify(1, ptr, idx, val, q, q, 1.0)
+    b = np.where(q > 0, 0.0, orhs)
+    return op, ptr, idx, val, b
+
+
+def _solve(op, b, method, tol=1e-8, true_res=False):
+    o = R.SolverOptions()
+    o.setSolverMethod(getattr(R.SolverOptions, method))
+    o.setTolerance(tol)
+    o.setTrueResidualCriterion(true_res)
+    return op.solve(to_dev(b), o).cpu().numpy(), o
+
+
+@pytest.mark.parametrize("dim,ne", SIZES)
+@pytest.mark.parametrize("sym", [False, True])
+@pytest.mark.parametrize("method", ["PCG", "PCG_PLAIN", "MINRES"])
+def test_symmetric_methods_match_the_oracle(dim, ne, sym, method):
+    op, ptr, idx, val, b = _problem(dim, ne, sym)
+    x, o = _solve(op, b, method)
+    xo, dg, _, _ = O.solve(1, ptr, idx, val.copy(), b, tolerance=1e-8)
+    assert o.hasConverged()
+    assert np.linalg.norm(x - xo) <= 1e-6 * np.linalg.norm(xo)
+    r = b - O.spmv(1, ptr, idx, val, x)
+    assert np.linalg.norm(r) <= 1e-6 * np.linalg.norm(b)
+    if method == "PCG":
+        n = o.getDiagnostics("num_iter")
+        assert abs(n - dg["num_iter"]) <= max(2, 0.02 * dg["num_iter"])
+
+
+@pytest.mark.parametrize("dim,ne", SIZES)
+def test_bicgstab_solves(dim, ne):
+    rng = np.random.default_rng(11 + sum(ne))
+    dom, length = grid(dim, ne)
+    E = dom.getNumElements()
+    c = {"A": np.exp(0.5 * rng.standard_normal(E))[:, None, None] * np.eye(dim)[None],
+         "C": 2.0 * rng.standard_normal((E, dim)), "D": rng.uniform(1.0, 2.0, E), "Y": rng.standard_normal(E)}
+    op, rhs = gpu_assemble(dom, 1, **c)
+    q = dirichlet_mask(dom, dim - 1)
+    op.nullifyRowsAndCols(to_dev(q), to_dev(q), 1.0)
+    ptr, idx, val, orhs = O.assemble(dim, ne, length, **c)
+    O.nullify(1, ptr, idx, val, q, q, 1.0)
+    b = np.where(q > 0, 0.0, orhs)
+    x, o = _solve(op, b, "BICGSTAB", tol=1e-10, true_res=True)
+    assert o.hasConverged()
+    r = b - O.spmv(1, ptr, idx, val, x)
+    assert np.linalg.norm(r) <= 2e-10 * np.linalg.norm(b)
+
+
+# the largest cube / square of each method's capacity (256 tiles of 512 x rows
+# per thread nodes) and the first beyond: the same solution to the tolerance
+@pytest.mark.parametrize("method,dim,n", [("PCG", 3, 70), ("PCG", 3, 76), ("PCG_PLAIN", 3, 70), ("MINRES", 3, 62),
+                                          ("MINRES", 3, 66), ("BICGSTAB", 3, 62), ("BICGSTAB", 3, 66),
+                                          ("PCG", 2, 700), ("PCG", 2, 740)])
+def test_capacity_edges(method, dim, n):
+    ne = (n,) * dim if dim == 2 else (n, n - 1, n - 3)
+    dom, _ = grid(dim, ne)
+    E, Q = dom.getNumElements(), 1 << dim
+    g = torch.Generator(device="cuda").manual_seed(n)
+    kap = torch.exp(torch.randn(E, dtype=torch.float64, device="cuda", generator=g) * 0.5)
+
+    def system():
+        op = dom.newOperator(1, symmetric=method != "BICGSTAB")
+        rhs = torch.zeros(op.size, dtype=torch.float64, device="cuda")
+        op.assemble({"A": R.Coefficient(kap, (dim, dim), E, Q, dom.device, isotropic=True),
+                     "Y": R.Coefficient(1.0, (), E, Q, dom.device)}, rhs)
+        q = dom.whereZero(dim - 1)
+        op.nullifyRowsAndCols(q, q, 1.0)
+        return op, torch.where(q > 0, torch.zeros_like(rhs), rhs)
+
+    op, b = system()
+    o = R.SolverOptions()
+    o.setSolverMethod(getattr(R.SolverOptions, method))
+    o.setTrueResidualCriterion(True)
+    x = op.solve(b, o)
+    op2, r = system()
+    op2.MatrixVector(-1.0, x, 1.0, r)
+    assert o.hasConverged()
+    assert (torch.linalg.norm(r) / torch.linalg.norm(b)).item() <= 1e-8
+
+
+def test_repeats_are_bit_identical_and_streams_do_not_matter():
+    op, ptr, idx, val, b = _problem(3, (30, 23, 17), True)
+    x1, _ = _solve(op, b, "PCG")
+    s = torch.cuda.Stream()
+    with torch.cuda.stream(s):
+        x2, _ = _solve(op, b, "PCG")
+    assert np.array_equal(x1, x2)
+
+
+@pytest.mark.parametrize("dim,ne", [(2, (44, 43)), (2, (97, 61)), (3, (10, 9, 11)), (3, (30, 23, 17))])
+@pytest.mark.parametrize("method", ["PCG", "PCG_PLAIN", "MINRES", "BICGSTAB"])
+def test_iteration_limits_match_the_launch_sequence(dim, ne, method):
+    # a check_interval selects the launch sequence; after k iterations both
+    # hold the same iterate but for the rounding of their sums
+    for k in (1, 2, 3, 4, 9, 17):
+        got = []
+        for interval in (0, 4):
+            op, _, _, _, b = _problem(dim, ne, True)
+            o = R.SolverOptions()
+            o.setSolverMethod(getattr(R.SolverOptions, method))
+            o.setTolerance(1e-12)
+            o.setIterMax(k)
+            o.setAcceptanceConvergenceFailureOn()
+            o.setCheckInterval(interval)
+            got.append((op.solve(to_dev(b), o).cpu().numpy(), o.getDiagnostics("num_iter"), o.hasConverged()))
+        assert got[0][1:] == got[1][1:]
+        assert np.linalg.norm(got[0][0] - got[1][0]) <= 1e-11 * np.linalg.norm(got[1][0])
+
+
+@pytest.mark.parametrize("method", ["PCG", "PCG_PLAIN", "MINRES", "BICGSTAB"])
+def test_special_right_hand_sides(method):
+    # zero, one that a multiple of the start vector solves at once, and the
+    # iterates of a system whose solution is reached in one step
+    dom, _ = grid(3, (6, 5, 7))
+    op, _ = gpu_assemble(dom, 1, symmetric=True, D=np.ones(dom.getNumElements()))
+    q = np.ones(op.size)
+    op.nullifyRowsAndCols(to_dev(q), to_dev(q), 2.0)     # the matrix is 2 I
+    b = np.random.default_rng(1).standard_normal(op.size)
+    o = R.SolverOptions()
+    o.setSolverMethod(getattr(R.SolverOptions, method))
+    assert np.array_equal(op.solve(to_dev(0 * b), o).cpu().numpy(), 0 * b)
+    x = op.solve(to_dev(b), o).cpu().numpy()
+    assert o.hasConverged() and np.allclose(x, 0.5 * b, rtol=1e-14, atol=0)
