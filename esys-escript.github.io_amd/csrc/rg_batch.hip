@@ -29,6 +29,7 @@
 #include "rg_device.h"
 #include "rg_dispatch.h"
 #include "rg_krylov.h"
+#include "rg_resident.h"
 #include "rg_stencil.h"
 
 namespace rg {
@@ -1122,31 +1123,41 @@ int batch_status(const rg_diagnostics* dg, int count, bool accept)
     return worst;
 }
 
-// Jacobi inverse (unbalanced) and, for FP32 values, the FP32 copy.
-void prepare_matrix(rg_matrix* m, bool fp32, double* dinv)
+// Jacobi inverses (unbalanced; of mats[j] at dinv + off[j]) and, for FP32
+// values, the FP32 copies.
+void prepare_matrices(rg_matrix* const* mats, size_t count, const int64_t* off, bool fp32, double* dinv)
 {
-    const Geom& g = m->g;
-    RG_CHECK(!m->is_balanced, RG_STATE_ERROR,
-             "batched solve: the matrix was balanced by an earlier solve; set or reset its values first");
-    hipStream_t st = m->ctx->stream;
+    for (size_t j = 0; j < count; ++j)
+        RG_CHECK(!mats[j]->is_balanced, RG_STATE_ERROR,
+                 "batched solve: the matrix was balanced by an earlier solve; set or reset its values first");
+    hipStream_t st = mats[0]->ctx->stream;
     DevArray<int> flag;
     flag.alloc(1);
     RG_HIP(hipMemsetAsync(flag.p, 0, sizeof(int), st));
-    const int center = (g.dim == 3 ? 27 : 9) / 2;
-    hipLaunchKernelGGL(k_diag_inv, dim3(std::min<int64_t>((g.N + 255) / 256, 4096)), dim3(256), 0, st, m->val, g.ld,
-                       g.N, center, dinv, flag.p);
+    for (size_t j = 0; j < count; ++j) {
+        const Geom& g = mats[j]->g;
+        const int center = (g.dim == 3 ? 27 : 9) / 2;
+        hipLaunchKernelGGL(k_diag_inv, dim3(std::min<int64_t>((g.N + 255) / 256, 4096)), dim3(256), 0, st, mats[j]->val,
+                           g.ld, g.N, center, dinv + off[j], flag.p);
+    }
     RG_HIP(hipGetLastError());
     int failed = 0;
     RG_HIP(hipMemcpyAsync(&failed, flag.p, sizeof(int), hipMemcpyDeviceToHost, st));
     RG_HIP(hipStreamSynchronize(st));
     RG_CHECK(!failed, RG_VALUE_ERROR, "batched solve: zero on the main diagonal");
-    if (fp32 && !m->val32_valid) {
-        if (!m->val32) {
-            RG_HIP(hipMalloc(&m->val32, value_count(m->g) * sizeof(float)));
-        }
+    for (size_t j = 0; fp32 && j < count; ++j) {
+        rg_matrix* m = mats[j];
+        if (m->val32_valid) continue;
+        if (!m->val32) RG_HIP(hipMalloc(&m->val32, value_count(m->g) * sizeof(float)));
         launch_to_fp32(m);
         m->val32_valid = true;
     }
+}
+
+void prepare_matrix(rg_matrix* m, bool fp32, double* dinv)
+{
+    const int64_t off = 0;
+    prepare_matrices(&m, 1, &off, fp32, dinv);
 }
 
 template <class F>
@@ -1558,6 +1569,7 @@ struct rg_batch {
     int built_mult = -1;
     bool built_fp32 = false;
     rg::ChunkRunner run;
+    rg::ResidentBatch resident;
 };
 
 namespace rg {
@@ -1661,7 +1673,7 @@ void batch_prepare(rg_batch* B, bool fp32)
 {
     const int64_t tot = B->offsets.back();
     B->dinv.alloc(tot);
-    for (size_t j = 0; j < B->mats.size(); ++j) prepare_matrix(B->mats[j], fp32, B->dinv.p + B->offsets[j]);
+    prepare_matrices(B->mats.data(), B->mats.size(), B->offsets.data(), fp32, B->dinv.p);
     B->r.alloc(tot);
     B->p.alloc(tot);
     B->q.alloc(tot);
@@ -1715,6 +1727,20 @@ int batch_solve(rg_batch* B, double* X, const double* b, const rg_options& opt, 
              "batch_solve: one Jacobi sweep is the only preconditioner");
     RG_CHECK(opt.tolerance > 0.0 && opt.tolerance <= 1.0, RG_VALUE_ERROR, "batch_solve: tolerance must be in (0, 1]");
     const bool fp32 = opt.method == RG_METHOD_PCG_MIXED;
+    // in one launch where every system fits in the registers (FP64 values,
+    // whatever the method asks of the product); a caller that gives a
+    // check_interval gets the launch sequence, whose replacements and polls
+    // it sets
+    if (opt.check_interval <= 0 && B->resident.plan(B->mats)) {
+        batch_prepare(B, false);
+        std::vector<KrylovState> fin;
+        if (B->resident.solve(B->mats, B->offsets, B->dinv.p, b, X, B->r.p, B->p.p, B->sts.p, opt.iter_max,
+                              opt.tolerance, 16 * kResSpins, fin)) {
+            fill_diagnostics(fin, now_s() - t0, dg, count);
+            return batch_status(dg, count, opt.accept_failed_convergence != 0);
+        }
+        B->resident.state = 2;
+    }
     if (B->tile_mult <= 0) batch_autotune(B, fp32, 5, nullptr);
     batch_prepare(B, fp32);
     if (B->built_mult != B->tile_mult || B->built_fp32 != fp32) build_tiles(B, B->tile_mult, fp32);

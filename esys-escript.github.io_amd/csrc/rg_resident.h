@@ -1,6 +1,8 @@
 // Krylov solves of small scalar systems in one launch (rg_resident.hip).
 #pragma once
 
+#include <vector>
+
 #include "rg_dispatch.h"
 #include "rg_internal.h"
 
@@ -14,14 +16,34 @@ constexpr unsigned kResSpins = 1u << 20;
 // sweep); false if it does not fit in the chip's registers or the method has
 // no such form.
 bool resident_fits(const rg_matrix* m, int method, int (&t)[3]);
-// As resident_fits, for any grid: at most `rows` nodes and `cells` padded
-// cells per tile, at most `tiles` tiles.
-bool resident_tiles(int dim, const int64_t* nn, int rows, int cells, int tiles, int (&t)[3]);
 size_t resident_slot_bytes();
 // Runs the Krylov loop from work->r, work->xw; work->xw is the new iterate.
 // False (xw then any iterate) if the launch was refused or a workgroup gave
 // up waiting for the others.
 bool resident_solve(rg_matrix* m, int method, const int (&t)[3], int maxit, double tol, unsigned spins,
                     KrylovState* out);
+
+// Many independent scalar systems (full storage, one dimension, one context)
+// by the textbook Jacobi-PCG in one launch.
+struct ResidentBatch {
+    int state = 0;               // 0 not looked at, 1 every system fits, 2 not
+    int grid = 0;                // workgroups
+    std::vector<int> tile;       // sides per system
+    std::vector<int> tiles;      // tiles per system
+    std::vector<int> first;      // tasks of each workgroup
+    std::vector<int32_t> tasks;  // (system, rank) pairs
+    void* mem = nullptr;         // device copies and slots
+
+    ResidentBatch() = default;
+    ResidentBatch(const ResidentBatch&) = delete;
+    ResidentBatch& operator=(const ResidentBatch&) = delete;
+    ~ResidentBatch();
+    bool plan(const std::vector<rg_matrix*>& mats);
+    // x from x = 0; off: the systems' offsets in dinv, b, x and the two work
+    // vectors.  False if the launch was refused or a workgroup gave up.
+    bool solve(const std::vector<rg_matrix*>& mats, const std::vector<int64_t>& off, const double* dinv, const double* b,
+               double* x, double* pub0, double* pub1, KrylovState* st, int maxit, double tol, unsigned spins,
+               std::vector<KrylovState>& out);
+};
 
 }  // namespace rg

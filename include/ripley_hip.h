@@ -395,7 +395,11 @@ int rg_multi_set_shape(rg_matrix* m, int shape);
  * free) solved together: every kernel launch spans all systems (a tile
  * table maps workgroups to (system, rows)).  Vectors are the systems'
  * vectors concatenated at rg_batch_offsets (count + 1 entries, each offset
- * a multiple of 64).  The matrices are borrowed. */
+ * a multiple of 64).  The matrices are borrowed.  Where every system fits on
+ * the chip and no check_interval is given, rg_batch_solve runs in one launch
+ * with FP64 values throughout (also for RG_METHOD_PCG_MIXED), takes the
+ * recursive residual to a tenth of the tolerance and then decides on
+ * ||b - A x||_2. */
 int rg_batch_create(rg_context* ctx, int count, rg_matrix* const* mats, rg_batch** out);
 int rg_batch_destroy(rg_batch* b);
 int rg_batch_offsets(const rg_batch* b, int64_t* offsets);

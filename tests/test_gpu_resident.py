@@ -153,3 +153,73 @@ def test_special_right_hand_sides(method):
     assert np.array_equal(op.solve(to_dev(0 * b), o).cpu().numpy(), 0 * b)
     x = op.solve(to_dev(b), o).cpu().numpy()
     assert o.hasConverged() and np.allclose(x, 0.5 * b, rtol=1e-14, atol=0)
+
+
+def _batch(shapes, seed, spread=0.7):
+    rng = np.random.default_rng(seed)
+    ops, vals, rhs = [], [], []
+    for ne in shapes:
+        dim = len(ne)
+        dom, length = grid(dim, ne)
+        E = dom.getNumElements()
+        A = np.exp(spread * rng.standard_normal(E))[:, None, None] * np.eye(dim)[None]
+        op, b = gpu_assemble(dom, 1, A=A, Y=rng.uniform(0.5, 1.5, E))
+        q = to_dev(dirichlet_mask(dom, 0))
+        op.nullifyRowsAndCols(q, q, 1.0)
+        ops.append(op)
+        rhs.append(torch.where(q > 0, torch.zeros_like(b), b))
+        vals.append(op.exportCSR())
+    return ops, vals, rhs
+
+
+# one tile each, many tiles, more tiles than the chip holds at once, one
+# system larger than all others, and the smallest grids
+BATCHES = [[(5, 3)], [(54, 54), (55, 55), (56, 54)], [(300, 290), (40, 700), (3, 3), (120, 64)],
+           [(260, 250)] * 6 + [(64, 64)] * 9, [(10, 11, 9)] * 3, [(40, 33, 37), (5, 4, 3), (1, 1, 900), (24, 24, 24)]]
+
+
+@pytest.mark.parametrize("shapes", BATCHES, ids=lambda s: "%d systems" % len(s))
+@pytest.mark.parametrize("method", ["PCG_PLAIN", "PCG_MIXED"])
+def test_batches_match_the_launch_sequence(shapes, method):
+    from ripley_hip import batch as RB
+    ops, vals, rhs = _batch(shapes, len(shapes))
+    solver = RB.BatchSolver(ops)
+    b = solver.join(rhs)
+    got = []
+    for interval in (0, 8):
+        o = R.SolverOptions()
+        o.setSolverMethod(getattr(R.SolverOptions, method))
+        o.setTolerance(1e-9)
+        o.setCheckInterval(interval)
+        x, diags = solver.solve(b, o)
+        assert all(d["converged"] for d in diags)
+        got.append(solver.split(x))
+    for (ptr, idx, val), x, y, f in zip(vals, got[0], got[1], rhs):
+        f = f.cpu().numpy()
+        r = f - O.spmv(1, ptr, idx, val, x.cpu().numpy())
+        assert np.linalg.norm(r) <= 1e-9 * (1 + 1e-6) * np.linalg.norm(f)
+        assert torch.linalg.norm(x - y) <= 1e-6 * torch.linalg.norm(y)
+
+
+def test_batch_limits_zero_sides_and_reuse():
+    from ripley_hip import batch as RB
+    ops, vals, rhs = _batch([(30, 30), (200, 90), (9, 9)], 5)
+    solver = RB.BatchSolver(ops)
+    o = R.SolverOptions()
+    o.setSolverMethod(R.SolverOptions.PCG_PLAIN)
+    o.setAcceptanceConvergenceFailureOn()
+    o.setIterMax(7)
+    rhs[2] = torch.zeros_like(rhs[2])
+    b = solver.join(rhs)
+    x7, diags = solver.solve(b, o)
+    assert [d["num_iter"] for d in diags] == [7, 7, 0]
+    assert [d["converged"] for d in diags] == [False, False, True]
+    o.setCheckInterval(7)
+    y7, _ = solver.solve(b, o)
+    assert torch.linalg.norm(x7 - y7) <= 1e-11 * torch.linalg.norm(y7)
+    o.setCheckInterval(0)
+    o.setIterMax(100000)
+    x, diags = solver.solve(b, o)
+    again, _ = solver.solve(b, o)
+    assert all(d["converged"] for d in diags) and torch.equal(x, again)
+    assert torch.count_nonzero(solver.split(x)[2]) == 0
