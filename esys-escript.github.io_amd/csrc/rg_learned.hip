@@ -316,20 +316,22 @@ __global__ __launch_bounds__(256) void k_conv_wgrad(Grid3 g, const bf16* __restr
         for (int j = 0; j < NTI; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
     for (int64_t vs = v0; vs < v1; vs += 128) {
         __syncthreads();
-        // stage: element e of (128 voxels x C) handled by thread t
-        for (int e = threadIdx.x; e < 128 * CIN; e += 256) {
-            const int vv = e / CIN, c = e % CIN;
+        // stage: 8 channels of one voxel per load, transposed into LDS
+        for (int e = threadIdx.x; e < 128 * (CIN / 8); e += 256) {
+            const int vv = e / (CIN / 8), c = 8 * (e % (CIN / 8));
             const int64_t v = vs + vv;
-            bf16 val = (bf16)0.f;
-            if (v < v1) val = in[(padded_index(gg, v) + off) * CIN + c];
-            xs[c][vv] = val;
+            bf16x8 val = {};
+            if (v < v1) val = *reinterpret_cast<const bf16x8*>(in + (padded_index(gg, v) + off) * CIN + c);
+#pragma unroll
+            for (int j = 0; j < 8; ++j) xs[c + j][vv] = val[j];
         }
-        for (int e = threadIdx.x; e < 128 * COUT; e += 256) {
-            const int vv = e / COUT, c = e % COUT;
+        for (int e = threadIdx.x; e < 128 * (COUT / 8); e += 256) {
+            const int vv = e / (COUT / 8), c = 8 * (e % (COUT / 8));
             const int64_t v = vs + vv;
-            bf16 val = (bf16)0.f;
-            if (v < v1) val = dy[padded_index(gg, v) * COUT + c];
-            ys[c][vv] = val;
+            bf16x8 val = {};
+            if (v < v1) val = *reinterpret_cast<const bf16x8*>(dy + padded_index(gg, v) * COUT + c);
+#pragma unroll
+            for (int j = 0; j < 8; ++j) ys[c + j][vv] = val[j];
         }
         __syncthreads();
         const int kv = 32 * wave + 8 * q;
@@ -358,57 +360,93 @@ __global__ __launch_bounds__(256) void k_conv_wgrad(Grid3 g, const bf16* __restr
             for (int r = 0; r < 4; ++r) dst[(16 * i + 4 * q + r) * CIN + 16 * jn + n] = acc[i][jn][r];
 }
 
-// dW[co][tap][ci] = sum over np partials of part[p][tap][co][ci] (fixed order),
-// and db[co] from the bias partials when given.
-__global__ void k_sum_wgrad(const float* __restrict__ part, int np, int cout, int cin, float* __restrict__ dw)
+// Sum of the np partials p[0], p[stride], ... in index order; the loads of 16
+// partials are issued before the first add (one at a time, a chain of 256
+// memory latencies took 60 us per layer of the 17^3 network, 540 of its 2070
+// us per gradient).
+__device__ __forceinline__ float sum_partials(const float* __restrict__ p, int np, int64_t stride)
+{
+    float s = 0.f;
+    int k = 0;
+    for (; k + 16 <= np; k += 16) {
+        float v[16];
+#pragma unroll
+        for (int u = 0; u < 16; ++u) v[u] = p[(k + u) * stride];
+#pragma unroll
+        for (int u = 0; u < 16; ++u) s += v[u];
+    }
+    for (; k < np; ++k) s += p[k * stride];
+    return s;
+}
+
+// dW[co][tap][ci] = sum over np partials of part[p][tap][co][ci], and db[co] =
+// sum over nb partials of bpart[p][co] (fixed order).
+__global__ void k_sum_grads(const float* __restrict__ part, int np, int cout, int cin, float* __restrict__ dw,
+                            const float* __restrict__ bpart, int nb, float* __restrict__ db)
 {
     const int64_t total = (int64_t)27 * cout * cin;
-    for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < total; e += (int64_t)gridDim.x * blockDim.x) {
-        const int ci = e % cin, co = (e / cin) % cout, tap = e / ((int64_t)cin * cout);
-        float s = 0.f;
-        for (int p = 0; p < np; ++p) s += part[(((int64_t)p * 27 + tap) * cout + co) * cin + ci];
-        dw[((int64_t)co * 27 + tap) * cin + ci] = s;
+    for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < total + cout;
+         e += (int64_t)gridDim.x * blockDim.x) {
+        if (e < total) {
+            const int ci = e % cin, co = (e / cin) % cout, tap = e / ((int64_t)cin * cout);
+            dw[((int64_t)co * 27 + tap) * cin + ci] = sum_partials(part + e, np, total);
+        } else {
+            db[e - total] = sum_partials(bpart + (e - total), nb, cout);
+        }
     }
 }
 
-// db[co] = sum_v dy[v][co]: per-block partials (fixed order), then summed.
-__global__ void k_bias_grad_part(Grid3 g, const bf16* __restrict__ dy, int cout, float* __restrict__ part,
-                                 int64_t vox_per_block)
+// db[co] = sum_v dy[v][co]: partials of voxel chunk blockIdx.x, channels
+// 8 blockIdx.y ..+8.  Thread t adds voxels t, t + 256, ...; then a tree over
+// the threads per channel: two levels from LDS, the rest by lane shifts (one
+// barrier for 8 channels; a barrier per level and channel took 34 us a layer).
+__global__ __launch_bounds__(256) void k_bias_grad_part(Grid3 g, const bf16* __restrict__ dy, int cout,
+                                                        float* __restrict__ part, int64_t vox_per_block)
 {
-    __shared__ float red[256];
+    __shared__ float red[8][256];
     const int64_t v0 = (int64_t)blockIdx.x * vox_per_block;
     int64_t v1 = v0 + vox_per_block;
     if (v1 > g.nvox) v1 = g.nvox;
-    for (int co = 0; co < cout; ++co) {
-        float s = 0.f;
-        for (int64_t v = v0 + threadIdx.x; v < v1; v += 256) s += (float)dy[padded_index(g, v) * cout + co];
-        red[threadIdx.x] = s;
-        __syncthreads();
-        for (int o = 128; o > 0; o >>= 1) {
-            if (threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
-            __syncthreads();
-        }
-        if (threadIdx.x == 0) part[(int64_t)blockIdx.x * cout + co] = red[0];
-        __syncthreads();
+    const int c0 = 8 * blockIdx.y, t = threadIdx.x, lane = t & 63, w = t >> 6;
+    float s[8] = {};
+    for (int64_t v = v0 + t; v < v1; v += 256) {
+        const bf16x8 d = *reinterpret_cast<const bf16x8*>(dy + padded_index(g, v) * cout + c0);
+#pragma unroll
+        for (int c = 0; c < 8; ++c) s[c] += (float)d[c];
+    }
+#pragma unroll
+    for (int c = 0; c < 8; ++c) red[c][t] = s[c];
+    __syncthreads();
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        const int c = 2 * w + h;
+        float v = (red[c][lane] + red[c][lane + 128]) + (red[c][lane + 64] + red[c][lane + 192]);
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) v += __shfl_down(v, o, 64);
+        if (lane == 0) part[(int64_t)blockIdx.x * cout + c0 + c] = v;
     }
 }
 
-__global__ void k_sum_rows(const float* __restrict__ part, int np, int n, float* __restrict__ out)
+// W^T with flipped taps for the data gradients, all layers in one launch:
+// wt[ci][tap][co] = w[co][26-tap][ci].
+constexpr int kMaxFlip = 16;
+struct FlipArgs {
+    const bf16* w[kMaxFlip];
+    bf16* wt[kMaxFlip];
+    int cin[kMaxFlip], cout[kMaxFlip];
+    int64_t first[kMaxFlip + 1];   // first element of each layer
+    int layers;
+};
+__global__ void k_flip_weights(FlipArgs a)
 {
-    for (int e = blockIdx.x * blockDim.x + threadIdx.x; e < n; e += gridDim.x * blockDim.x) {
-        float s = 0.f;
-        for (int p = 0; p < np; ++p) s += part[(int64_t)p * n + e];
-        out[e] = s;
-    }
-}
-
-// W^T with flipped taps for the data gradient: wt[ci][tap][co] = w[co][26-tap][ci].
-__global__ void k_flip_weights(const bf16* __restrict__ w, int cout, int cin, bf16* __restrict__ wt)
-{
-    const int64_t total = (int64_t)27 * cout * cin;
-    for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < total; e += (int64_t)gridDim.x * blockDim.x) {
+    for (int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; g < a.first[a.layers];
+         g += (int64_t)gridDim.x * blockDim.x) {
+        int l = 0;
+        while (g >= a.first[l + 1]) ++l;
+        const int64_t e = g - a.first[l];
+        const int cout = a.cout[l], cin = a.cin[l];
         const int co = e % cout, tap = (e / cout) % 27, ci = e / ((int64_t)cout * 27);
-        wt[((int64_t)ci * 27 + tap) * cout + co] = w[((int64_t)co * 27 + (26 - tap)) * cin + ci];
+        a.wt[l][((int64_t)ci * 27 + tap) * cout + co] = a.w[l][((int64_t)co * 27 + (26 - tap)) * cin + ci];
     }
 }
 
@@ -667,11 +705,18 @@ void conv_fwd(hipStream_t st, const Grid3& g, int cin, int cout, const bf16* in,
     throw Error(RG_VALUE_ERROR, "conv: unsupported channel pair");
 }
 
+// Voxels per workgroup of the weight gradient: at most nchunk workgroups per
+// tap, multiples of 128 voxels (the coarse levels then have fewer chunks).
+inline int64_t wgrad_chunk(const Grid3& g, int nchunk)
+{
+    return ((g.nvox + nchunk - 1) / nchunk + 127) / 128 * 128;
+}
+
 template <int CIN, int COUT>
 void conv_wgrad_t(hipStream_t st, const Grid3& g, const bf16* x, const bf16* dy, float* part, int nchunk)
 {
-    const int64_t vpb = ((g.nvox + nchunk - 1) / nchunk + 127) / 128 * 128;
-    hipLaunchKernelGGL((k_conv_wgrad<CIN, COUT>), dim3(nchunk, 27), dim3(256), 0, st, g, x, dy, part, vpb);
+    const int64_t vpb = wgrad_chunk(g, nchunk);
+    hipLaunchKernelGGL((k_conv_wgrad<CIN, COUT>), dim3((unsigned)((g.nvox + vpb - 1) / vpb), 27), dim3(256), 0, st, g, x, dy, part, vpb);
 }
 
 void conv_wgrad(hipStream_t st, const Grid3& g, int cin, int cout, const bf16* x, const bf16* dy, float* part,
@@ -698,7 +743,7 @@ struct Net {
     std::vector<float*> W32, B32;  // FP32 master parameters (device)
     std::vector<bf16*> W16;        // BF16 weights used by the convolutions
     std::vector<bf16*> WT16;       // flipped/transposed weights for data gradients
-    std::vector<float*> gW, gB;    // gradients
+    std::vector<float*> gW, gB;    // gradients, one allocation in parameter order
     std::vector<float*> mW, vW, mB, vB;   // Adam moments
     int adam_t = 0;
     // activations (forward) and their gradients (backward)
@@ -750,8 +795,8 @@ void net_init(Net& N, rg_context* ctx, const int32_t* nodes, bool training)
         N.W16.push_back((bf16*)N.alloc(sizeof(bf16) * ws));
         if (training) {
             N.WT16.push_back((bf16*)N.alloc(sizeof(bf16) * ws));
-            N.gW.push_back((float*)N.alloc(sizeof(float) * ws));
-            N.gB.push_back((float*)N.alloc(sizeof(float) * kLayers[l].cout));
+            N.gW.push_back(l == 0 ? (float*)N.alloc(sizeof(float) * total_params()) : N.gB[l - 1] + kLayers[l - 1].cout);
+            N.gB.push_back(N.gW[l] + ws);
             N.mW.push_back((float*)N.alloc(sizeof(float) * ws));
             N.vW.push_back((float*)N.alloc(sizeof(float) * ws));
             N.mB.push_back((float*)N.alloc(sizeof(float) * kLayers[l].cout));
@@ -773,7 +818,7 @@ void net_init(Net& N, rg_context* ctx, const int32_t* nodes, bool training)
         int64_t mx = 0;
         for (int l = 0; l < kNumLayers; ++l) mx = std::max<int64_t>(mx, layer_wsize(l));
         N.part_elems = (int64_t)N.nchunk * 4 * mx;
-        N.part = (float*)N.alloc(sizeof(float) * N.part_elems);
+        N.part = (float*)N.alloc(sizeof(float) * (N.part_elems + (int64_t)N.nchunk * 64));   // + bias partials
     }
     N.scale = (double*)N.alloc(sizeof(double) * 4);
     N.red = (double*)N.alloc(sizeof(double) * (3 * 1024 + 8));   // partials, then 3 loss dots at 3*1024
@@ -953,15 +998,20 @@ __global__ void k_loss_part(Grid3 g, int n0, int n1, int n2, const bf16* __restr
         for (int k = 0; k < 3; ++k) part[k * gridDim.x + blockIdx.x] = red[k][0];
 }
 
-__global__ void k_loss_final(const double* __restrict__ part, int np, double* __restrict__ out)
+// The three sums of np <= 256 partials each, in index order (from LDS: read
+// one at a time from memory they took 42 us).
+__global__ __launch_bounds__(256) void k_loss_final(const double* __restrict__ part, int np, double* __restrict__ out)
 {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
-    double s[3] = {0.0, 0.0, 0.0};
+    __shared__ double p[3][256];
     for (int k = 0; k < 3; ++k)
-        for (int b = 0; b < np; ++b) s[k] += part[k * np + b];
-    out[0] = s[0];
-    out[1] = s[1];
-    out[2] = s[2];
+        if ((int)threadIdx.x < np) p[k][threadIdx.x] = part[k * np + threadIdx.x];
+    __syncthreads();
+    if (threadIdx.x < 3) {
+        double s = 0.0;
+#pragma unroll 16
+        for (int b = 0; b < np; ++b) s += p[threadIdx.x][b];
+        out[threadIdx.x] = s;
+    }
 }
 
 __global__ void k_loss_grad(Grid3 g, int n0, int n1, int n2, const bf16* __restrict__ y, const double* __restrict__ e,
@@ -1041,11 +1091,12 @@ void layer_wgrad(Net& N, int l, const Grid3& g, const bf16* x, const bf16* dpre)
     hipStream_t st = N.ctx->stream;
     const int cin = kLayers[l].cin, cout = kLayers[l].cout;
     conv_wgrad(st, g, cin, cout, x, dpre, N.part, N.nchunk);
-    hipLaunchKernelGGL(k_sum_wgrad, dim3(ew_grid(layer_wsize(l))), dim3(256), 0, st, N.part, N.nchunk * 4, cout, cin,
-                       N.gW[l]);
     const int64_t vpb = (g.nvox + N.nchunk - 1) / N.nchunk;
-    hipLaunchKernelGGL(k_bias_grad_part, dim3(N.nchunk), dim3(256), 0, st, g, dpre, cout, N.part, vpb);
-    hipLaunchKernelGGL(k_sum_rows, dim3(1), dim3(256), 0, st, N.part, N.nchunk, cout, N.gB[l]);
+    float* bpart = N.part + N.part_elems;
+    hipLaunchKernelGGL(k_bias_grad_part, dim3(N.nchunk, cout / 8), dim3(256), 0, st, g, dpre, cout, bpart, vpb);
+    const int64_t wpb = wgrad_chunk(g, N.nchunk);
+    hipLaunchKernelGGL(k_sum_grads, dim3(ew_grid(layer_wsize(l) + cout)), dim3(256), 0, st, N.part,
+                       4 * (int)((g.nvox + wpb - 1) / wpb), cout, cin, N.gW[l], bpart, N.nchunk, N.gB[l]);
 }
 
 // dx = conv^T(dpre) with the flipped weights of layer l (cout -> cin channels)
@@ -1053,8 +1104,6 @@ void layer_dgrad(Net& N, int l, const Grid3& g, const bf16* dpre, bf16* dx)
 {
     hipStream_t st = N.ctx->stream;
     const int cin = kLayers[l].cin, cout = kLayers[l].cout;
-    hipLaunchKernelGGL(k_flip_weights, dim3(ew_grid(layer_wsize(l))), dim3(256), 0, st, N.W16[l], cout, cin,
-                       N.WT16[l]);
     conv_fwd(st, g, cout, cin, dpre, N.WT16[l], nullptr, dx, false);
 }
 
@@ -1073,16 +1122,28 @@ double net_gradients(Net& N, const double* r, const double* dinv, const float* l
     net_forward(N, r, dinv, nullptr, logk, energy ? N.zbuf : nullptr, st, true);
     const int np = 256;
     RG_HIP(hipMemsetAsync(N.gy.p, 0, sizeof(bf16) * padded_size(g1) * 16, st));
+    // layers 1.. (the data gradient of layer 0 is not needed)
+    FlipArgs fa;
+    fa.layers = kNumLayers - 1;
+    fa.first[0] = 0;
+    for (int l = 1; l < kNumLayers; ++l) {
+        fa.w[l - 1] = N.W16[l];
+        fa.wt[l - 1] = N.WT16[l];
+        fa.cin[l - 1] = kLayers[l].cin;
+        fa.cout[l - 1] = kLayers[l].cout;
+        fa.first[l] = fa.first[l - 1] + layer_wsize(l);
+    }
+    hipLaunchKernelGGL(k_flip_weights, dim3(ew_grid(fa.first[fa.layers])), dim3(256), 0, st, fa);
     if (energy) {
         launch_spmv_on(N.loss_op, 1.0, N.zbuf, 0.0, N.azbuf, st);
         hipLaunchKernelGGL(k_energy_part, dim3(np), dim3(256), 0, st, nn, r, N.zbuf, N.azbuf, e, N.red);
-        hipLaunchKernelGGL(k_loss_final, dim3(1), dim3(64), 0, st, N.red, np, N.red + 3 * 1024);
+        hipLaunchKernelGGL(k_loss_final, dim3(1), dim3(256), 0, st, N.red, np, N.red + 3 * 1024);
         hipLaunchKernelGGL(k_energy_grad, dim3(ew_grid(nn)), dim3(256), 0, st, g1, N.n[0], N.n[1], N.n[2], r,
                            N.azbuf, N.red + 3 * 1024, N.scale, N.gy.p);
     } else {
         // cosine loss on the output in normalised units (the output is y / scale)
         hipLaunchKernelGGL(k_loss_part, dim3(np), dim3(256), 0, st, g1, N.n[0], N.n[1], N.n[2], N.y.p, e, N.red);
-        hipLaunchKernelGGL(k_loss_final, dim3(1), dim3(64), 0, st, N.red, np, N.red + 3 * 1024);
+        hipLaunchKernelGGL(k_loss_final, dim3(1), dim3(256), 0, st, N.red, np, N.red + 3 * 1024);
         hipLaunchKernelGGL(k_loss_grad, dim3(ew_grid(nn)), dim3(256), 0, st, g1, N.n[0], N.n[1], N.n[2], N.y.p, e,
                            N.red + 3 * 1024, N.gy.p);
     }
@@ -1295,15 +1356,8 @@ int rg_lpc_gradients(rg_lpc* h, const double* r, const double* dinv, const float
         const double L = rg::lpc::net_gradients(N, r, dinv, logk, e);
         if (loss) *loss = L;
         if (grads) {
-            int64_t o = 0;
-            for (int l = 0; l < rg::lpc::kNumLayers; ++l) {
-                const int64_t ws = rg::lpc::layer_wsize(l);
-                RG_HIP(hipMemcpyAsync(grads + o, N.gW[l], ws * sizeof(float), hipMemcpyDeviceToHost, N.ctx->stream));
-                o += ws;
-                const int co = rg::lpc::kLayers[l].cout;
-                RG_HIP(hipMemcpyAsync(grads + o, N.gB[l], co * sizeof(float), hipMemcpyDeviceToHost, N.ctx->stream));
-                o += co;
-            }
+            RG_HIP(hipMemcpyAsync(grads, N.gW[0], rg::lpc::total_params() * sizeof(float), hipMemcpyDeviceToHost,
+                                  N.ctx->stream));
             RG_HIP(hipStreamSynchronize(N.ctx->stream));
         }
         return RG_OK;
