@@ -184,7 +184,7 @@ __host__ __device__ constexpr int asm_nodes_per_wave()
 // quadrature points and the one-point rule (GAUSS = true) take the Gauss sum,
 // the point loop outermost so that the shape functions of a point serve all
 // elements.  Both in one kernel took 256 registers (one wave per SIMD); a PDE
-// with both kinds runs one launch of each.
+// with both kinds runs a launch of each.
 //
 // Bound: the coefficient reads.  A data point of a system is NB^2 DIM^2 (A)
 // contiguous doubles of which thread (k, m) needs every NB-th, so the lanes
@@ -193,7 +193,7 @@ __host__ __device__ constexpr int asm_nodes_per_wave()
 // four waves take 2 x 2 neighbouring node lines (3-D; four lines in 2-D),
 // which share their elements through L1.  With one (k, m) per blockIdx.y and
 // lanes along x, each load touched 64 lines: Brick 48x47x49, 3 equations,
-// A per element and the rest on quadrature points 10.48 ms -> 0.17 + 1.09 ms (bytes alone 0.24 ms);
+// A per element and the rest on quadrature points 10.48 ms -> 0.17 + 1.00 ms (bytes alone 0.24 ms);
 // Brick 96^3 elasticity (A per element, symmetric storage) 37.6 -> 0.92 ms (bytes alone 0.30 ms).
 template <int DIM, int NB>
 struct AsmNode {
@@ -361,23 +361,62 @@ __global__ __launch_bounds__(kBlock) void k_assemble_const(AsmArgs a, double* __
     if (doF) rhs[nd.i * NB + k] += f;
 }
 
-template <int DIM, int NB, bool SYM>
+// The Gauss sum of a group of coefficients: A alone (AGROUP), or B, C, D, X, Y.
+// For each quadrature point the block stages its elements' points of the
+// group in LDS (a thread per double, whole runs of a data point; zeros for
+// elements outside the grid), and every node reads its 2^DIM elements from
+// there (each double once per block and point instead of once per node
+// through L1): B, C, D, X, Y of three equations on Brick 48x47x49 1.09 ->
+// 1.00 ms, C, D, Y of one on Brick 63x64x40 167 -> 94 us (bytes alone 0.12
+// ms and 13 us; the rest is staging, LDS reads and sums one after the other).
+template <int DIM, int NB>
+struct AsmBlock {
+    static constexpr int EX = asm_nodes_per_wave<NB>() + 1;   // elements of the block along each axis
+    static constexpr int EY = DIM == 3 ? 3 : 5;
+    static constexpr int EZ = DIM == 3 ? 3 : 1;
+    static constexpr int ELEMENTS = EX * EY * EZ;
+    static constexpr int dpsA = NB * DIM * NB * DIM, dpsB = NB * DIM * NB, dpsD = NB * NB, dpsX = NB * DIM, dpsY = NB;
+    // doubles per element of each group
+    static constexpr int A_SIZE = dpsA, REST_SIZE = 2 * dpsB + dpsD + dpsX + dpsY;
+};
+
+template <int DIM, int NB, bool SYM, bool AGROUP>
 __global__ __launch_bounds__(kBlock) void k_assemble_gauss(AsmArgs a, double* __restrict__ val, int64_t ld,
                                                            int64_t tiles_x, int64_t tiles_y, bool zero,
                                                            double* __restrict__ rhs)
 {
+    using Blk = AsmBlock<DIM, NB>;
     constexpr int NS = StencilShape<DIM>::NS;
     constexpr int NNODE = 1 << DIM;
+    constexpr int PER = AGROUP ? Blk::A_SIZE : Blk::REST_SIZE;
+    constexpr int oB = 0, oC = Blk::dpsB, oD = 2 * Blk::dpsB, oX = oD + Blk::dpsD, oY = oX + Blk::dpsX;
+    __shared__ double lds[Blk::ELEMENTS * PER];
     const AsmNode<DIM, NB> nd(a, tiles_x, tiles_y);
-    if (!nd.valid) return;
     const int k = nd.k, m = nd.m;
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     const double ih[3] = {1.0 / a.h0, 1.0 / a.h1, 1.0 / a.h2};
     double vol = a.h0 * a.h1;
     if (DIM == 3) vol *= a.h2;
-    const bool doS = (a.A.mode | a.B.mode | a.C.mode | a.D.mode) != 0;
-    const bool doF = rhs != nullptr && m == 0 && (a.X.mode | a.Y.mode) != 0;
-    constexpr int dpsA = NB * DIM * NB * DIM, dpsB = NB * DIM * NB, dpsC = NB * NB * DIM, dpsD = NB * NB;
-    constexpr int dpsX = NB * DIM, dpsY = NB;
+    const bool doS = AGROUP || (a.B.mode | a.C.mode | a.D.mode) != 0;
+    const bool doF = !AGROUP && rhs != nullptr && m == 0 && (a.X.mode | a.Y.mode) != 0;
+    // the block's element (0, 0, 0)
+    const int64_t bx = blockIdx.x % tiles_x, by = (blockIdx.x / tiles_x) % tiles_y, bz = blockIdx.x / (tiles_x * tiles_y);
+    const int64_t fx = bx * (Blk::EX - 1) - 1, fy = by * (Blk::EY - 1) - 1, fz = DIM == 3 ? bz * (Blk::EZ - 1) - 1 : 0;
+    // the points of quadrature point q of one coefficient, DPS doubles each
+    auto stage = [&](const CoefDev& c, auto dps, int offset, int q) {
+        constexpr int DPS = decltype(dps)::value;
+        if (!c.mode) return;
+        const int point = (AGROUP && c.iso) ? 1 : DPS;   // an isotropic A stages its scalar only
+        for (int idx = threadIdx.x; idx < Blk::ELEMENTS * DPS; idx += kBlock) {
+            const int el = idx / DPS, o = idx % DPS;
+            if (o >= point) continue;
+            const int64_t k0 = fx + el % Blk::EX, k1 = fy + (el / Blk::EX) % Blk::EY, k2 = fz + el / (Blk::EX * Blk::EY);
+            const bool in = k0 >= 0 && k0 < a.ne0 && k1 >= 0 && k1 < a.ne1 && (DIM == 2 || (k2 >= 0 && k2 < a.ne2));
+            double v = 0.0;
+            if (in) v = coef_pt(c, k0 + (int64_t)a.ne0 * (k1 + (int64_t)a.ne1 * k2), q, point)[o];
+            lds[el * PER + offset + o] = v;
+        }
+    };
     double acc[NS];
 #pragma unroll
     for (int s = 0; s < NS; ++s) acc[s] = 0.0;
@@ -385,8 +424,22 @@ __global__ __launch_bounds__(kBlock) void k_assemble_gauss(AsmArgs a, double* __
     const int nq = a.reduced ? 1 : NNODE;
     const double w = vol / nq;
     const double g0 = 0.5 - 0.5 / 1.73205080756887719318, g1 = 0.5 + 0.5 / 1.73205080756887719318;
+    // element t of the node in LDS
+    const int e0 = (min(lane / (NB * NB), Blk::EX - 2) +
+                    Blk::EX * (DIM == 3 ? (wv & 1) + Blk::EY * (wv >> 1) : wv)) * PER;
 #pragma unroll 1
     for (int q = 0; q < nq; ++q) {
+        __syncthreads();
+        if constexpr (AGROUP) {
+            stage(a.A, IC<Blk::dpsA>{}, 0, q);
+        } else {
+            stage(a.B, IC<Blk::dpsB>{}, oB, q);
+            stage(a.C, IC<Blk::dpsB>{}, oC, q);
+            stage(a.D, IC<Blk::dpsD>{}, oD, q);
+            stage(a.X, IC<Blk::dpsX>{}, oX, q);
+            stage(a.Y, IC<Blk::dpsY>{}, oY, q);
+        }
+        __syncthreads();
         double phi[DIM][2];   // 1-D shape functions at the point
 #pragma unroll
         for (int p = 0; p < DIM; ++p) {
@@ -417,62 +470,57 @@ __global__ __launch_bounds__(kBlock) void k_assemble_gauss(AsmArgs a, double* __
         };
 #pragma unroll
         for (int t = 0; t < NNODE; ++t) {
-            if (nd.in & (1u << t)) {
-                // opaque per use: the addresses of all elements' points, kept
-                // over the point loop, took 100 registers
-                int64_t e = nd.element(a, t);
-                asm volatile("" : "+v"(e));
-                const int la = (NNODE - 1) - t;   // the node's local index in element t
-                double u[DIM], c0 = 0.0;
+            const double* P = lds + e0 + ((t & 1) + Blk::EX * (((t >> 1) & 1) + Blk::EY * (t >> 2))) * PER;
+            const int la = (NNODE - 1) - t;   // the node's local index in element t
+            double u[DIM], c0 = 0.0;
 #pragma unroll
-                for (int j = 0; j < DIM; ++j) u[j] = 0.0;
-                if (a.A.mode) {
-                    const double* P = coef_pt(a.A, e, q, a.A.iso ? 1 : dpsA);
-                    if (a.A.iso) {
+            for (int j = 0; j < DIM; ++j) u[j] = 0.0;
+            if constexpr (AGROUP) {
+                if (a.A.iso) {
 #pragma unroll
-                        for (int j = 0; j < DIM; ++j) u[j] = P[0] * G(la, j);
-                    } else {
+                    for (int j = 0; j < DIM; ++j) u[j] = P[0] * G(la, j);
+                } else {
 #pragma unroll
-                        for (int j = 0; j < DIM; ++j)
+                    for (int j = 0; j < DIM; ++j)
 #pragma unroll
-                            for (int p = 0; p < DIM; ++p)
-                                u[j] = fma(P[k + NB * (p + DIM * (m + NB * j))], G(la, p), u[j]);
-                    }
+                        for (int p = 0; p < DIM; ++p)
+                            u[j] = fma(P[k + NB * (p + DIM * (m + NB * j))], G(la, p), u[j]);
                 }
+            } else {
                 if (a.C.mode) {
-                    const double* P = coef_pt(a.C, e, q, dpsC);
 #pragma unroll
-                    for (int j = 0; j < DIM; ++j) u[j] = fma(P[k + NB * (m + NB * j)], N[la], u[j]);
+                    for (int j = 0; j < DIM; ++j) u[j] = P[oC + k + NB * (m + NB * j)] * N[la];
                 }
                 if (a.B.mode) {
-                    const double* P = coef_pt(a.B, e, q, dpsB);
 #pragma unroll
-                    for (int p = 0; p < DIM; ++p) c0 = fma(P[k + NB * (p + DIM * m)], G(la, p), c0);
+                    for (int p = 0; p < DIM; ++p) c0 = fma(P[oB + k + NB * (p + DIM * m)], G(la, p), c0);
                 }
-                if (a.D.mode) c0 = fma(coef_pt(a.D, e, q, dpsD)[k + NB * m], N[la], c0);
-                if (doS) {
+                if (a.D.mode) c0 = fma(P[oD + k + NB * m], N[la], c0);
+            }
+            if (doS) {
 #pragma unroll
-                    for (int b = 0; b < NNODE; ++b) {
-                        const int s = asm_slot<DIM>(t, b);
-                        if (SYM && s < StencilShape<DIM>::CENTER) continue;
-                        double r = fma(c0, N[b], acc[s]);
+                for (int b = 0; b < NNODE; ++b) {
+                    const int s = asm_slot<DIM>(t, b);
+                    if (SYM && s < StencilShape<DIM>::CENTER) continue;
+                    double r = AGROUP ? acc[s] : fma(c0, N[b], acc[s]);
+                    if (AGROUP || a.C.mode) {
 #pragma unroll
                         for (int j = 0; j < DIM; ++j) r = fma(u[j], G(b, j), r);
-                        acc[s] = r;
                     }
+                    acc[s] = r;
                 }
-                if (doF) {
-                    if (a.X.mode) {
-                        const double* P = coef_pt(a.X, e, q, dpsX);
+            }
+            if (doF) {
+                if (a.X.mode) {
 #pragma unroll
-                        for (int p = 0; p < DIM; ++p) f = fma(P[k + NB * p], G(la, p), f);
-                    }
-                    if (a.Y.mode) f = fma(coef_pt(a.Y, e, q, dpsY)[k], N[la], f);
+                    for (int p = 0; p < DIM; ++p) f = fma(P[oX + k + NB * p], G(la, p), f);
                 }
+                if (a.Y.mode) f = fma(P[oY + k], N[la], f);
             }
             __builtin_amdgcn_sched_barrier(0);
         }
     }
+    if (!nd.valid) return;
     if (doS) {
 #pragma unroll
         for (int s = 0; s < NS; ++s) acc[s] *= w;
@@ -797,12 +845,11 @@ void launch_assemble(rg_matrix* m, const rg_pde_coefs& c, int reduced, double* r
         AsmArgs ac = a, ag = a;
         CoefDev* const both[6][2] = {{&ac.A, &ag.A}, {&ac.B, &ag.B}, {&ac.C, &ag.C},
                                      {&ac.D, &ag.D}, {&ac.X, &ag.X}, {&ac.Y, &ag.Y}};
-        bool is_const = false, is_gauss = false;
+        bool is_const = false;
         for (auto& p : both) {
             const int mode = p[0]->mode;
             const bool cst = !reduced && mode == RG_COEF_ELEMENT;
             is_const = is_const || cst;
-            is_gauss = is_gauss || (mode && !cst);
             p[cst ? 1 : 0]->mode = RG_COEF_EMPTY;
         }
         dispatch(g, m->symmetric, [&](auto D, auto B, auto S) {
@@ -818,9 +865,14 @@ void launch_assemble(rg_matrix* m, const rg_pde_coefs& c, int reduced, double* r
                                    ac, m->val, g.ld, tx, ty, zero, rhs);
                 if (ac.A.mode || ac.B.mode || ac.C.mode || ac.D.mode) zero = false;
             }
-            if (is_gauss)
-                hipLaunchKernelGGL((k_assemble_gauss<D.value, B.value, S.value>), grid, dim3(kBlock), 0, m->ctx->stream,
-                                   ag, m->val, g.ld, tx, ty, zero, rhs);
+            if (ag.A.mode) {
+                hipLaunchKernelGGL((k_assemble_gauss<D.value, B.value, S.value, true>), grid, dim3(kBlock), 0,
+                                   m->ctx->stream, ag, m->val, g.ld, tx, ty, zero, rhs);
+                zero = false;
+            }
+            if (ag.B.mode || ag.C.mode || ag.D.mode || ag.X.mode || ag.Y.mode)
+                hipLaunchKernelGGL((k_assemble_gauss<D.value, B.value, S.value, false>), grid, dim3(kBlock), 0,
+                                   m->ctx->stream, ag, m->val, g.ld, tx, ty, zero, rhs);
         });
     }
     RG_HIP(hipGetLastError());
