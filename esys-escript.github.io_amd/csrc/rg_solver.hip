@@ -21,6 +21,7 @@
 #include "rg_device.h"
 #include "rg_dispatch.h"
 #include "rg_krylov.h"
+#include "rg_march.h"
 #include "rg_mg.h"
 #include "rg_resident.h"
 #include "rg_stencil.h"
@@ -28,6 +29,9 @@
 namespace rg {
 
 namespace {
+
+// MI355X's memory-side cache (Infinity Cache, MALL).
+constexpr int64_t kMallBytes = 256ll << 20;
 
 double now_s()
 {
@@ -480,6 +484,34 @@ __global__ __launch_bounds__(kBlock) void k_spmv_dot(PcgArgs a, const VT* __rest
                                         }
                                     });
     publish_block_sums<1>(dl, a.partials);
+}
+
+// k_spmv_dot for symmetric block storage by marching in z (Brick 96^3, 3 x 3
+// blocks, 920 MB of values: 285 -> 220 us, 4.2 TB/s).
+template <int BS, typename VT>
+__global__ __launch_bounds__(kMarchThreads) void k_spmv_dot_march(PcgArgs a, MarchArgs g, const VT* __restrict__ val)
+{
+    if (a.st->done) return;
+    double* __restrict__ v = a.v;
+    double dl = 0.0;
+    const int block = (int)xcd_block();
+    if (block < march_blocks(g))
+        march_block<BS, VT>(g, block, val, a.ld, a.p, [&](int64_t i, const double (&y)[BS], const double (&p)[BS]) {
+#pragma unroll
+            for (int r = 0; r < BS; ++r) {
+                v[i * BS + r] = y[r];
+                dl = fma(y[r], p[r], dl);
+            }
+        });
+    __shared__ double red[kMarchThreads / 64];
+    dl = wave_sum(dl);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = dl;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        double t = 0.0;
+        for (int w = 0; w < kMarchThreads / 64; ++w) t += red[w];
+        a.partials[blockIdx.x] = t;
+    }
 }
 
 // a.N counts scalar entries here (nodes * block size).
@@ -1023,6 +1055,37 @@ struct SolverImpl {
     Launch spmv_launch() const { return chunked_launch(m->g.N, spmv_rows_per_thread<VT>()); }
     Launch node_launch() const { return chunked_launch(m->g.N, m->g.bs == 1 ? 2 : 1); }
 
+    // v = A p with the partials of p.v; returns their number.
+    template <typename VT, bool PASO>
+    int spmv_dot(const PcgArgs& asp, int grid, const VT* val)
+    {
+        const Geom& g = m->g;
+        const MarchArgs ma = g.dim == 3 && g.bs == 3 ? march_args(g, m->ctx->num_cu) : MarchArgs{};
+        if (marches(ma, sizeof(VT))) {
+            hipLaunchKernelGGL((k_spmv_dot_march<3, VT>), dim3(march_grid(ma)), dim3(kMarchThreads), 0, st, asp, ma, val);
+            return march_grid(ma);
+        }
+        dispatch(g, m->symmetric, [&](auto D, auto B, auto S) {
+            hipLaunchKernelGGL((k_spmv_dot<D.value, B.value, S.value, VT, PASO>), dim3(grid), dim3(kBlock), 0, st, asp,
+                               val);
+        });
+        return grid;
+    }
+    // Whether the product marches (rg_march.h): symmetric storage of 3 x 3
+    // blocks on a Brick whose values do not fit in the MALL; below that the
+    // gather kernel's transposed re-reads come from there.  Layered
+    // elasticity on n^3 elements, whole PASO solves gather / march: n = 56
+    // (FP64 values, 187 MB) 49.3 / 54.2 ms, 60 (229 MB) 65.9 / 73.7, 64
+    // (277 MB) 94.6 / 87.5, 72 (392 MB) 134 / 119, 96 (920 MB) 403 / 337; FP32
+    // values 64 (138 MB) 63.1 / 67.5, 80 (268 MB) 149 / 125, 96 (460 MB) 280 /
+    // 266.  Thin grids without a tile for at least every other CU gather.
+    bool marches(const MarchArgs& ma, size_t vsize) const
+    {
+        const Geom& g = m->g;
+        return m->symmetric && g.dim == 3 && g.bs == 3 && (int64_t)(g.N * vsize) < ((int64_t)1 << 32) &&
+               (int64_t)g.nstore * 9 * g.ld * (int64_t)vsize > kMallBytes && 2 * march_blocks(ma) >= m->ctx->num_cu;
+    }
+
     // z = M^-1 r with `sweeps` Jacobi sweeps, into w->z (returns the buffer).
     double* jacobi(const double* r, int sweeps, const KrylovState* guard)
     {
@@ -1079,13 +1142,11 @@ struct SolverImpl {
         PcgArgs ar = args(zb, chunked_launch(g.N * g.bs, 2));
         ar.N = g.N * g.bs;
         const Launch Lr = chunked_launch(ar.N, 2);
-        dispatch(g, m->symmetric, [&](auto D, auto B, auto S) {
+        dispatch_bs(g.bs, [&](auto B) {
             hipLaunchKernelGGL((k_p_update<B.value, double, false, NT>), dim3(Ln.grid), dim3(kBlock), 0, st, an,
                                m->dinv);
-            hipLaunchKernelGGL((k_spmv_dot<D.value, B.value, S.value, double, true>), dim3(Lsp.grid), dim3(kBlock), 0,
-                               st, asp, m->val);
         });
-        stage<ST_PASO_SPMV, 1>(Lsp.grid);
+        stage<ST_PASO_SPMV, 1>(spmv_dot<double, true>(asp, Lsp.grid, m->val));
         // gamma's reduction folded into k_paso_x (both on the fold shape):
         // 128^3 Brick, full storage 0.2676 -> 0.2632 s per PASO solve; with
         // the non-temporal streams of symmetric storage 0.2004 -> 0.2012 s,
@@ -1156,18 +1217,17 @@ struct SolverImpl {
         af.partials = m->ctx->partials + 8 * kMaxGrid;   // rows 8.. of the partials: untouched by the SpMV
         af.fold_partials = af.partials;
         af.fold_G = Lf.grid;
+        const int parts = spmv_dot<VT, false>(asp, Lsp.grid, val);
         dispatch(g, m->symmetric, [&](auto D, auto B, auto S) {
-            hipLaunchKernelGGL((k_spmv_dot<D.value, B.value, S.value, VT, false>), dim3(Lsp.grid), dim3(kBlock), 0,
-                               st, asp, val);
             if (fd) {
-                stage<ST_CGX_SPMV, 1>(Lsp.grid);
+                stage<ST_CGX_SPMV, 1>(parts);
                 hipLaunchKernelGGL((k_cg_update<B.value, DT, true, NT>), dim3(Lf.grid), dim3(kBlock), 0, st, af, dinv);
             } else if (xd) {
-                stage<ST_CGX_SPMV, 1>(Lsp.grid);
+                stage<ST_CGX_SPMV, 1>(parts);
                 hipLaunchKernelGGL((k_cg_update<B.value, DT, true, NT>), dim3(Ln.grid), dim3(kBlock), 0, st, an, dinv);
                 stage<ST_CGX_UPDATE, 2>(Ln.grid);
             } else {
-                stage<ST_CG_SPMV, 1>(Lsp.grid);
+                stage<ST_CG_SPMV, 1>(parts);
                 hipLaunchKernelGGL((k_cg_update<B.value, DT, false, NT>), dim3(Ln.grid), dim3(kBlock), 0, st, an, dinv);
                 if (buf) stage<ST_CG_UPDATE_NORZ, 2>(Ln.grid);
                 else stage<ST_CG_UPDATE, 2>(Ln.grid);
@@ -1462,9 +1522,6 @@ struct SolverImpl {
         *nmax = m->ctx->pinned[1];
     }
 };
-
-// MI355X's memory-side cache (Infinity Cache, MALL).
-constexpr int64_t kMallBytes = 256ll << 20;
 
 // Whether the update kernels stream their vectors non-temporally: when the
 // SpMV's values fit in the MALL but values plus the vectors an iteration
