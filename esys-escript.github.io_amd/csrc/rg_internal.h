@@ -158,6 +158,7 @@ struct rg_matrix {
     double* balance = nullptr;     // N*bs balance vector
     bool is_balanced = false;
     bool have_prec = false;
+    bool unit_jacobi = false;      // the Jacobi inverse is 1 to rounding in every row
     bool val_zero = true;          // every stored value is known to be 0 (assembly may write instead of add)
     rg_solver_work* work = nullptr;
     int multi_shape = 0;           // SpMM tile shape + 1 of the many-RHS solver (0: autotune)

@@ -996,9 +996,10 @@ bool resident_solve(rg_matrix* m, int method, const int (&t)[3], int maxit, doub
                               sizeof(ResShared) <= 65536, "the tile outgrew the LDS");
         const unsigned lds = (unsigned)(sizeof(double) * (vecs * cells + own * rows));
         // all workgroups wait for one another: a cooperative launch starts
-        // them together or not at all
-        err = hipLaunchCooperativeKernel(reinterpret_cast<const void*>(k_resident<D.value, T.value>), dim3(tiles),
-                                         dim3(kResThreads), args, lds, st);
+        // them together or not at all (one alone needs none)
+        const void* kernel = reinterpret_cast<const void*>(k_resident<D.value, T.value>);
+        err = tiles == 1 ? hipLaunchKernel(kernel, dim3(1), dim3(kResThreads), args, lds, st)
+                         : hipLaunchCooperativeKernel(kernel, dim3(tiles), dim3(kResThreads), args, lds, st);
     });
     if (err != hipSuccess) {
         (void)hipGetLastError();

@@ -223,3 +223,45 @@ def test_batch_limits_zero_sides_and_reuse():
     again, _ = solver.solve(b, o)
     assert all(d["converged"] for d in diags) and torch.equal(x, again)
     assert torch.count_nonzero(solver.split(x)[2]) == 0
+
+
+# iterations whose streams exceed the L2s: the PCGs' update kernels leave the
+# Jacobi inverse unread where it is 1 to rounding (diffusion after PASO's
+# balance) and read it where it is not (element matrices whose off-diagonal
+# entries exceed a diagonal one); the one-launch solve always reads it
+@pytest.mark.parametrize("unit", [True, False])
+@pytest.mark.parametrize("method", ["PCG", "PCG_PLAIN"])
+def test_unread_jacobi_inverse(unit, method):
+    rng = np.random.default_rng(3)
+    got = []
+    if unit:
+        dom, _ = grid(3, (64, 65, 63))
+        A = np.exp(0.7 * rng.standard_normal(dom.getNumElements()))[:, None, None] * np.eye(3)[None]
+        make = lambda: gpu_assemble(dom, 1, symmetric=True, A=A)[0]
+    else:
+        n = 600
+        dom, _ = grid(2, (n, n))
+        ix = np.arange(n * n)
+        n0 = (ix % n) + (n + 1) * (ix // n)
+        nodes = np.stack([n0, n0 + 1, n0 + n + 1, n0 + n + 2], axis=1).astype(np.int32)
+        s = np.exp(1.0 * rng.standard_normal((n * n, 4)))
+        em = s[:, :, None] * (np.eye(4) + 0.8)[None] * s[:, None, :]
+
+        def make():
+            op = dom.newOperator(1)
+            op.addElementBlocks(nodes, em)
+            return op
+    b = rng.standard_normal(dom.getNumNodes())
+    for interval in (0, 32):
+        op = make()
+        if unit:
+            q = to_dev(dirichlet_mask(dom, 2))
+            op.nullifyRowsAndCols(q, q, 1.0)
+        o = R.SolverOptions()
+        o.setSolverMethod(getattr(R.SolverOptions, method))
+        o.setTolerance(1e-9)
+        o.setCheckInterval(interval)
+        got.append((op.solve(to_dev(b), o), o.getDiagnostics("num_iter")))
+        assert o.hasConverged()
+    assert abs(got[0][1] - got[1][1]) <= max(2, 0.02 * got[1][1])
+    assert torch.linalg.norm(got[0][0] - got[1][0]) <= 1e-7 * torch.linalg.norm(got[1][0])
