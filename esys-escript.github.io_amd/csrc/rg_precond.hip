@@ -342,7 +342,10 @@ struct SweepArgs {
 // acc -= sum over the stencil slots t != C of M(t) x[row + off_t], for the
 // split copies: entries outside the grid or of the other colour side are
 // zero, so only indices outside [0, N) need care (clamped and selected away).
-template <int DIM, int BS>
+// FRESH: x holds rows that nothing has been written to yet; their entries are
+// zero here, and what x holds there (uninitialised memory may read as NaN) is
+// not multiplied by them.
+template <int DIM, int BS, bool FRESH>
 __device__ __forceinline__ void split_product(const SweepArgs& a, const double* M, int64_t pos, int64_t row,
                                               const double* __restrict__ x, double (&acc)[BS])
 {
@@ -361,7 +364,10 @@ __device__ __forceinline__ void split_product(const SweepArgs& a, const double* 
 #pragma unroll
             for (int d = 0; d < 3; ++d) {
                 const int t = 3 * l + d;
-                if (t != C) acc[0] = fma(-ldg(&M[(int64_t)t * a.ld + pos]), xk[d], acc[0]);
+                if (t != C) {
+                    const double mv = ldg(&M[(int64_t)t * a.ld + pos]);
+                    acc[0] = fma(-mv, FRESH && mv == 0.0 ? 0.0 : xk[d], acc[0]);
+                }
             }
         }
         return;
@@ -383,7 +389,10 @@ __device__ __forceinline__ void split_product(const SweepArgs& a, const double* 
         for (int r = 0; r < BS; ++r) {
             double s = 0.0;
 #pragma unroll
-            for (int c = 0; c < BS; ++c) s = fma(mv[r + BS * c], xk[c], s);
+            for (int c = 0; c < BS; ++c) {
+                const double m = mv[r + BS * c];
+                s = fma(m, FRESH && m == 0.0 ? 0.0 : xk[c], s);
+            }
             acc[r] = in ? acc[r] - s : acc[r];
         }
     }
@@ -404,7 +413,7 @@ __global__ __launch_bounds__(kSweepBlock) void k_colour_forward(SweepArgs a, int
     double acc[BS];
 #pragma unroll
     for (int q = 0; q < BS; ++q) acc[q] = b[row * BS + q];
-    split_product<DIM, BS>(a, a.plow, pos, row, x, acc);
+    split_product<DIM, BS, true>(a, a.plow, pos, row, x, acc);
     double out[BS];
     block_mv<BS>(a.pdinv + pos, a.ld, acc, out);
 #pragma unroll
@@ -432,7 +441,7 @@ __global__ __launch_bounds__(kSweepBlock) void k_colour_backward(SweepArgs a, in
     } else {
         block_mv<BS>(a.pdiag + pos, a.ld, xi, acc);
     }
-    split_product<DIM, BS>(a, a.pup, pos, row, x, acc);
+    split_product<DIM, BS, false>(a, a.pup, pos, row, x, acc);
     if (ILU) {
 #pragma unroll
         for (int q = 0; q < BS; ++q) x[row * BS + q] = acc[q];

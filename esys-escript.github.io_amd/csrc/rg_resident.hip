@@ -44,7 +44,10 @@ constexpr int kResWaves = kResThreads / 64;
 constexpr int kMaxSums = 4;        // sums of one reduction
 constexpr int kSets = 4;           // sets of slots
 constexpr int kMaxTiles = 256;     // one per CU
-constexpr unsigned long long kEmpty = 0xFFF8DEADBEEF0001ull;   // a NaN no sum is stored as
+// An empty slot: a denormal (about 1e-309; a sum of these very bits is stored
+// as its neighbour).  A finite number, because freed slots become other
+// buffers' uninitialised memory.
+constexpr unsigned long long kEmpty = 0x0000DEADBEEF0001ull;
 
 // One system: its matrix, grid and tiling.
 struct ResSystem {
@@ -154,9 +157,10 @@ __device__ __forceinline__ bool reduce_all(ResShared& sh, const Gang& a, unsigne
             unsigned long long* nxt = a.slots + (size_t)((epoch + 2) & (kSets - 1)) * G * kMaxSums;
 #pragma unroll
             for (int k = 0; k < NV; ++k)
-                if (lane == k)
-                    put(cur + a.rank * kMaxSums + k,
-                        s[k] == s[k] ? (unsigned long long)__double_as_longlong(s[k]) : 0x7FF8000000000000ull);
+                if (lane == k) {
+                    const unsigned long long b = (unsigned long long)__double_as_longlong(s[k]);
+                    put(cur + a.rank * kMaxSums + k, b == kEmpty ? b ^ 1 : b);
+                }
             unsigned long long u[kMaxTiles / 64][NV];
             unsigned left = a.spins;
             do {
