@@ -193,7 +193,7 @@ __host__ __device__ constexpr int asm_nodes_per_wave()
 // four waves take 2 x 2 neighbouring node lines (3-D; four lines in 2-D),
 // which share their elements through L1.  With one (k, m) per blockIdx.y and
 // lanes along x, each load touched 64 lines: Brick 48x47x49, 3 equations,
-// A per element and the rest on quadrature points 10.48 ms -> 0.17 + 1.00 ms (bytes alone 0.24 ms);
+// A per element and the rest on quadrature points 10.48 ms -> 0.17 + 0.77 ms (bytes alone 0.24 ms);
 // Brick 96^3 elasticity (A per element, symmetric storage) 37.6 -> 0.92 ms (bytes alone 0.30 ms).
 template <int DIM, int NB>
 struct AsmNode {
@@ -367,8 +367,9 @@ __global__ __launch_bounds__(kBlock) void k_assemble_const(AsmArgs a, double* __
 // elements outside the grid), and every node reads its 2^DIM elements from
 // there (each double once per block and point instead of once per node
 // through L1): B, C, D, X, Y of three equations on Brick 48x47x49 1.09 ->
-// 1.00 ms, C, D, Y of one on Brick 63x64x40 167 -> 94 us (bytes alone 0.12
-// ms and 13 us; the rest is staging, LDS reads and sums one after the other).
+// 1.00 ms, and with the next point fetched during the sums 0.77 ms (bytes
+// alone 0.12 ms); C, D, Y of one on Brick 63x64x40 167 -> 94 us (bytes alone
+// 13 us).  What is left is LDS reads and sums in turn with two barriers a point.
 template <int DIM, int NB>
 struct AsmBlock {
     static constexpr int EX = asm_nodes_per_wave<NB>() + 1;   // elements of the block along each axis
@@ -399,22 +400,60 @@ __global__ __launch_bounds__(kBlock) void k_assemble_gauss(AsmArgs a, double* __
     if (DIM == 3) vol *= a.h2;
     const bool doS = AGROUP || (a.B.mode | a.C.mode | a.D.mode) != 0;
     const bool doF = !AGROUP && rhs != nullptr && m == 0 && (a.X.mode | a.Y.mode) != 0;
-    // the block's element (0, 0, 0)
-    const int64_t bx = blockIdx.x % tiles_x, by = (blockIdx.x / tiles_x) % tiles_y, bz = blockIdx.x / (tiles_x * tiles_y);
-    const int64_t fx = bx * (Blk::EX - 1) - 1, fy = by * (Blk::EY - 1) - 1, fz = DIM == 3 ? bz * (Blk::EZ - 1) - 1 : 0;
-    // the points of quadrature point q of one coefficient, DPS doubles each
-    auto stage = [&](const CoefDev& c, auto dps, int offset, int q) {
+    // grid index of each element of the block, -1 outside the grid
+    __shared__ int64_t index[Blk::ELEMENTS];
+    {
+        const int64_t bx = blockIdx.x % tiles_x, by = (blockIdx.x / tiles_x) % tiles_y,
+                      bz = blockIdx.x / (tiles_x * tiles_y);
+        for (int el = threadIdx.x; el < Blk::ELEMENTS; el += kBlock) {
+            const int64_t k0 = bx * (Blk::EX - 1) - 1 + el % Blk::EX,
+                          k1 = by * (Blk::EY - 1) - 1 + (el / Blk::EX) % Blk::EY,
+                          k2 = DIM == 3 ? bz * (Blk::EZ - 1) - 1 + el / (Blk::EX * Blk::EY) : 0;
+            const bool in = k0 >= 0 && k0 < a.ne0 && k1 >= 0 && k1 < a.ne1 && (DIM == 2 || (k2 >= 0 && k2 < a.ne2));
+            index[el] = in ? k0 + (int64_t)a.ne0 * (k1 + (int64_t)a.ne1 * k2) : -1;
+        }
+        __syncthreads();
+    }
+    // the points of quadrature point q of one coefficient, DPS doubles each:
+    // loaded into registers (ahead, see AHEAD), then stored
+    auto fetch = [&](const CoefDev& c, auto& v, auto dps, int q) {
         constexpr int DPS = decltype(dps)::value;
         if (!c.mode) return;
         const int point = (AGROUP && c.iso) ? 1 : DPS;   // an isotropic A stages its scalar only
-        for (int idx = threadIdx.x; idx < Blk::ELEMENTS * DPS; idx += kBlock) {
-            const int el = idx / DPS, o = idx % DPS;
-            if (o >= point) continue;
-            const int64_t k0 = fx + el % Blk::EX, k1 = fy + (el / Blk::EX) % Blk::EY, k2 = fz + el / (Blk::EX * Blk::EY);
-            const bool in = k0 >= 0 && k0 < a.ne0 && k1 >= 0 && k1 < a.ne1 && (DIM == 2 || (k2 >= 0 && k2 < a.ne2));
-            double v = 0.0;
-            if (in) v = coef_pt(c, k0 + (int64_t)a.ne0 * (k1 + (int64_t)a.ne1 * k2), q, point)[o];
-            lds[el * PER + offset + o] = v;
+        const double* p = c.p + (c.mode == RG_COEF_EXPANDED ? q * point : 0);
+        int tid = threadIdx.x;
+        if (AGROUP || NB == 1) asm volatile("" : "+v"(tid));   // addresses formed anew for each point: registers
+#pragma unroll
+        for (int u = 0; u < (Blk::ELEMENTS * DPS + kBlock - 1) / kBlock; ++u) {
+            const int idx = tid + u * kBlock, el = idx / DPS, o = idx % DPS;
+            v[u] = 0.0;
+            if (idx < Blk::ELEMENTS * DPS && o < point) {
+                const int64_t e = index[el];
+                if (e >= 0) v[u] = p[e * c.stride + o];
+            }
+        }
+    };
+    auto store = [&](const CoefDev& c, const auto& v, auto dps, int offset) {
+        constexpr int DPS = decltype(dps)::value;
+        if (!c.mode) return;
+#pragma unroll
+        for (int u = 0; u < (Blk::ELEMENTS * DPS + kBlock - 1) / kBlock; ++u) {
+            const int idx = threadIdx.x + u * kBlock;
+            if (idx < Blk::ELEMENTS * DPS) lds[idx / DPS * PER + offset + idx % DPS] = v[u];
+        }
+    };
+    constexpr auto trips = [](int dps) { return (Blk::ELEMENTS * dps + kBlock - 1) / kBlock; };
+    double fA[AGROUP ? trips(Blk::dpsA) : 1], fB[AGROUP ? 1 : trips(Blk::dpsB)], fC[AGROUP ? 1 : trips(Blk::dpsB)],
+        fD[AGROUP ? 1 : trips(Blk::dpsD)], fX[AGROUP ? 1 : trips(Blk::dpsX)], fY[AGROUP ? 1 : trips(Blk::dpsY)];
+    auto fetch_point = [&](int q) {
+        if constexpr (AGROUP) {
+            fetch(a.A, fA, IC<Blk::dpsA>{}, q);
+        } else {
+            fetch(a.B, fB, IC<Blk::dpsB>{}, q);
+            fetch(a.C, fC, IC<Blk::dpsB>{}, q);
+            fetch(a.D, fD, IC<Blk::dpsD>{}, q);
+            fetch(a.X, fX, IC<Blk::dpsX>{}, q);
+            fetch(a.Y, fY, IC<Blk::dpsY>{}, q);
         }
     };
     double acc[NS];
@@ -427,19 +466,26 @@ __global__ __launch_bounds__(kBlock) void k_assemble_gauss(AsmArgs a, double* __
     // element t of the node in LDS
     const int e0 = (min(lane / (NB * NB), Blk::EX - 2) +
                     Blk::EX * (DIM == 3 ? (wv & 1) + Blk::EY * (wv >> 1) : wv)) * PER;
+    // the next point's loads during the sums of this one: for systems other
+    // than A (A's points beside its sums took more than 256 registers; a
+    // single PDE's few doubles gain nothing: 94 -> 104 us)
+    constexpr bool AHEAD = !AGROUP && NB > 1;
+    if (AHEAD) fetch_point(0);
 #pragma unroll 1
     for (int q = 0; q < nq; ++q) {
         __syncthreads();
+        if (!AHEAD) fetch_point(q);
         if constexpr (AGROUP) {
-            stage(a.A, IC<Blk::dpsA>{}, 0, q);
+            store(a.A, fA, IC<Blk::dpsA>{}, 0);
         } else {
-            stage(a.B, IC<Blk::dpsB>{}, oB, q);
-            stage(a.C, IC<Blk::dpsB>{}, oC, q);
-            stage(a.D, IC<Blk::dpsD>{}, oD, q);
-            stage(a.X, IC<Blk::dpsX>{}, oX, q);
-            stage(a.Y, IC<Blk::dpsY>{}, oY, q);
+            store(a.B, fB, IC<Blk::dpsB>{}, oB);
+            store(a.C, fC, IC<Blk::dpsB>{}, oC);
+            store(a.D, fD, IC<Blk::dpsD>{}, oD);
+            store(a.X, fX, IC<Blk::dpsX>{}, oX);
+            store(a.Y, fY, IC<Blk::dpsY>{}, oY);
         }
         __syncthreads();
+        if (AHEAD && q + 1 < nq) fetch_point(q + 1);
         double phi[DIM][2];   // 1-D shape functions at the point
 #pragma unroll
         for (int p = 0; p < DIM; ++p) {
