@@ -21,6 +21,7 @@
 #include <string>
 #include <vector>
 
+#include "rg_plan.h"
 #include "ripley_hip.h"
 
 namespace rg {
@@ -43,8 +44,6 @@ struct Error : std::runtime_error {
     } while (0)
 
 constexpr int kBlock = 256;          // threads per workgroup of every streaming kernel
-constexpr int kNumXcd = 8;           // MI355X: 8 XCDs, blocks dispatched round-robin
-constexpr int kMaxGrid = 8192;       // grid cap of chunked streaming kernels (partials per reduction)
 // Size of the per-device scratch array of the allocation-free entry points.
 constexpr int64_t kScratchBytes = RG_SCRATCH_BYTES;
 

@@ -16,18 +16,10 @@
 #pragma once
 
 #include "rg_device.h"
+#include "rg_plan.h"
 #include "rg_stencil.h"
 
 namespace rg {
-
-constexpr int kMarchThreads = 512;   // nodes of a tile and its ring
-
-struct MarchArgs {
-    int n0, n1, n2;
-    int tx, ty;          // tile sides
-    int gx, gy;          // tiles per plane
-    int zs;              // planes per segment
-};
 
 // Barrier for LDS data: loads from memory stay in flight.
 __device__ __forceinline__ void lds_barrier()
@@ -151,43 +143,5 @@ __device__ __forceinline__ void march_block(const MarchArgs& g, int block, const
         }
     }
 }
-
-// Tiling of a grid for march_block: tiles of at most kMarchThreads nodes with
-// their ring, and z segments so that `want` workgroups are reached.
-inline MarchArgs march_args(const Geom& g, int want)
-{
-    MarchArgs m;
-    m.n0 = (int)g.nn[0];
-    m.n1 = (int)g.nn[1];
-    m.n2 = (int)g.nn[2];
-    // least loaded area: nodes plus the ring's share of blocks (9 of 14 along each side)
-    double best = 1e300;
-    for (int gx = 1; gx <= m.n0; ++gx) {
-        const int tx = (m.n0 + gx - 1) / gx;
-        if (tx + 2 > kMarchThreads / 3 || (m.n0 + tx - 1) / tx != gx) continue;
-        int ty = kMarchThreads / (tx + 2) - 2;
-        if (ty < 1) continue;
-        if (ty > m.n1) ty = m.n1;
-        const int gy = (m.n1 + ty - 1) / ty;
-        ty = (m.n1 + gy - 1) / gy;
-        const double area = gx * gy * (tx * ty + 9.0 / 14.0 * (tx + ty));
-        if (area < best) {
-            best = area;
-            m.tx = tx;
-            m.ty = ty;
-            m.gx = gx;
-            m.gy = gy;
-        }
-    }
-    int segs = std::max(1, want / (m.gx * m.gy));
-    segs = std::min(segs, std::max(1, m.n2 / 4));
-    m.zs = (m.n2 + segs - 1) / segs;
-    return m;
-}
-// Tiles x segments, and the workgroups launched for them: a multiple of the
-// XCDs, so that xcd_block puts neighbouring tiles, which share the memory
-// lines at their edges, on one XCD.
-__host__ __device__ inline int march_blocks(const MarchArgs& m) { return m.gx * m.gy * ((m.n2 + m.zs - 1) / m.zs); }
-inline int march_grid(const MarchArgs& m) { return (march_blocks(m) + kNumXcd - 1) / kNumXcd * kNumXcd; }
 
 }  // namespace rg

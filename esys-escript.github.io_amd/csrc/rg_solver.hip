@@ -30,9 +30,7 @@ namespace rg {
 
 namespace {
 
-// MI355X's memory-side cache (Infinity Cache, MALL).
-constexpr int64_t kMallBytes = 256ll << 20;
-constexpr int64_t kL2Bytes = 32ll << 20;   // its eight L2s together
+constexpr int64_t kL2Bytes = 32ll << 20;   // MI355X's eight L2s together
 
 double now_s()
 {
@@ -1091,30 +1089,19 @@ struct SolverImpl {
     int spmv_dot(const PcgArgs& asp, int grid, const VT* val)
     {
         const Geom& g = m->g;
-        const MarchArgs ma = g.dim == 3 && g.bs == 3 ? march_args(g, m->ctx->num_cu) : MarchArgs{};
-        if (marches(ma, sizeof(VT))) {
-            hipLaunchKernelGGL((k_spmv_dot_march<3, VT>), dim3(march_grid(ma)), dim3(kMarchThreads), 0, st, asp, ma, val);
-            return march_grid(ma);
+        if (g.dim == 3 && g.bs == 3 && m->symmetric) {
+            const MarchArgs ma = march_args((int)g.nn[0], (int)g.nn[1], (int)g.nn[2], m->ctx->num_cu);
+            if (march_applies(ma, (int64_t)g.nstore * 9 * g.ld * (int64_t)sizeof(VT), sizeof(VT), m->ctx->num_cu)) {
+                const int blocks = (int)march_grid(ma);
+                hipLaunchKernelGGL((k_spmv_dot_march<3, VT>), dim3(blocks), dim3(kMarchThreads), 0, st, asp, ma, val);
+                return blocks;
+            }
         }
         dispatch(g, m->symmetric, [&](auto D, auto B, auto S) {
             hipLaunchKernelGGL((k_spmv_dot<D.value, B.value, S.value, VT, PASO>), dim3(grid), dim3(kBlock), 0, st, asp,
                                val);
         });
         return grid;
-    }
-    // Whether the product marches (rg_march.h): symmetric storage of 3 x 3
-    // blocks on a Brick whose values do not fit in the MALL; below that the
-    // gather kernel's transposed re-reads come from there.  Layered
-    // elasticity on n^3 elements, whole PASO solves gather / march: n = 56
-    // (FP64 values, 187 MB) 49.3 / 54.2 ms, 60 (229 MB) 65.9 / 73.7, 64
-    // (277 MB) 94.6 / 87.5, 72 (392 MB) 134 / 119, 96 (920 MB) 403 / 337; FP32
-    // values 64 (138 MB) 63.1 / 67.5, 80 (268 MB) 149 / 125, 96 (460 MB) 280 /
-    // 266.  Thin grids without a tile for at least every other CU gather.
-    bool marches(const MarchArgs& ma, size_t vsize) const
-    {
-        const Geom& g = m->g;
-        return m->symmetric && g.dim == 3 && g.bs == 3 && (int64_t)(g.N * vsize) < ((int64_t)1 << 32) &&
-               (int64_t)g.nstore * 9 * g.ld * (int64_t)vsize > kMallBytes && 2 * march_blocks(ma) >= m->ctx->num_cu;
     }
 
     // z = M^-1 r with `sweeps` Jacobi sweeps, into w->z (returns the buffer).

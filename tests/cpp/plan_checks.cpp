@@ -1,0 +1,57 @@
+// Rules of the launch plans (rg_plan.h), checked on the host: exit code 0 if
+// all hold, otherwise the failing rule is printed.
+#include <cstdio>
+
+#include "rg_plan.h"
+
+static int bad = 0;
+#define EXPECT(cond, ...)                \
+    do {                                 \
+        if (!(cond)) {                   \
+            std::printf(__VA_ARGS__);    \
+            std::printf(": %s\n", #cond); \
+            ++bad;                       \
+        }                                \
+    } while (0)
+
+// values of symmetric 3 x 3 blocks: 14 stored slots of 9 entries
+static bool marches(int e0, int e1, int e2, int vsize, int cu = 256)
+{
+    const rg::MarchArgs m = rg::march_args(e0 + 1, e1 + 1, e2 + 1, cu);
+    const int64_t ld = ((int64_t)(e0 + 1) * (e1 + 1) * (e2 + 1) + 63) / 64 * 64;
+    return rg::march_applies(m, 14 * 9 * ld * vsize, vsize, cu);
+}
+
+// the reducing kernels write one partial per workgroup: no plan has more of
+// them than partials (kMaxGrid)
+static void march_fits_the_partials()
+{
+    const int wide[][3] = {{7600, 7600, 1}, {1850, 1850, 20}, {2400, 1600, 3}, {60, 90000, 2}, {90000, 60, 2}, {3000, 3000, 4}};
+    for (auto& e : wide)
+        for (int vsize : {4, 8}) {
+            const rg::MarchArgs m = rg::march_args(e[0] + 1, e[1] + 1, e[2] + 1, 256);
+            EXPECT(!marches(e[0], e[1], e[2], vsize) || rg::march_grid(m) <= rg::kMaxGrid, "%d x %d x %d", e[0], e[1], e[2]);
+        }
+    EXPECT(!marches(7600, 7600, 1, 8), "137,922 workgroups");
+    EXPECT(marches(96, 96, 96, 8) && marches(96, 96, 96, 4) && marches(1400, 1300, 1, 8), "grids that march");
+}
+
+// every node belongs to one tile and segment, and a tile fits the workgroup
+static void march_covers()
+{
+    for (int n0 : {2, 3, 9, 65, 97, 170, 171, 700})
+        for (int n1 : {2, 14, 97, 513})
+            for (int n2 : {2, 5, 97, 9001}) {
+                const rg::MarchArgs m = rg::march_args(n0, n1, n2, 256);
+                EXPECT((m.tx + 2) * (m.ty + 2) <= rg::kMarchThreads, "%d x %d x %d", n0, n1, n2);
+                EXPECT((int64_t)m.tx * m.gx >= n0 && m.tx * (m.gx - 1) < n0, "%d x %d x %d", n0, n1, n2);
+                EXPECT((int64_t)m.ty * m.gy >= n1 && m.ty * (m.gy - 1) < n1, "%d x %d x %d", n0, n1, n2);
+            }
+}
+
+int main()
+{
+    march_fits_the_partials();
+    march_covers();
+    return bad != 0;
+}
