@@ -141,7 +141,11 @@ __device__ __forceinline__ bool reduce_all(ResShared& sh, const Gang& a, unsigne
         const double s = wave_total(v[k]);
         if (lane == 0) sh.red[k][w] = s;
     }
-    __builtin_amdgcn_s_waitcnt(0);   // this wave's surface values and emptied slots have arrived
+    // this wave's surface values and emptied slots have arrived before any slot
+    // is written (a memory clobber: the barrier's workgroup fence alone lets
+    // agent-scope stores be in flight, and a wait that does not name memory
+    // may be moved ahead of them)
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
     __syncthreads();
     if (w == 0) {
         double s[NV];
