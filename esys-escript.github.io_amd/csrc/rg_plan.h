@@ -67,15 +67,32 @@ constexpr int64_t march_grid(const MarchArgs& m) { return (march_blocks(m) + kNu
 // elements, whole PASO solves gather / march: n = 56 (FP64 values, 187 MB)
 // 49.3 / 54.2 ms, 60 (229 MB) 65.9 / 73.7, 64 (277 MB) 94.6 / 87.5, 72
 // (392 MB) 134 / 119, 96 (920 MB) 403 / 337; FP32 values 64 (138 MB) 63.1 /
-// 67.5, 80 (268 MB) 149 / 125, 96 (460 MB) 280 / 266.  Thin grids without a
-// tile for at least every other CU gather.  So do grids with more workgroups
-// than a reduction has partials (some 3.4 M nodes per plane; the gather
-// kernel's blocks take longer chunks instead).
+// 67.5, 80 (268 MB) 149 / 125, 96 (460 MB) 280 / 266.
+//
+// And only where tiles and segments use the chip.  A workgroup takes zs + 1
+// steps (planes), each a fixed time (27 barriers) and one per tile node; the
+// gather kernel takes a time per node of the grid.  SpMV alone, gather / march
+// in us, by N / (steps * (200 + tile nodes)) for FP64 values: 2x2x60000
+// elements 11: 192 / 1752, 8x8x9000 70: 251 / 421, 64x63x66 75: 97 / 108,
+// 228x228x30 83: 609 / 529, 66^3 85: 104 / 95, 64^3 94: 96 / 88, 96^3 138:
+// 301 / 231; tiles of 100 to 144 nodes lose by more than that says (10x10x7000
+// 91: 284 / 351, 11x11x5000 100: 245 / 262; 169 nodes, 12x12x4000 108: 238 /
+// 223).  FP32 values, whose loads of 40-byte runs and fixed time weigh
+// more, by the share of threads with a node, N / (steps * 512 * CUs):
+// 8x8x9000 0.15: 129 / 300, 228x228x30 0.39: 331 / 404, 30x30x900 0.41: 164 /
+// 202, 260x250x20 0.48: 281 / 265, 200x180x40 0.52: 298 / 265, 96^3 0.58:
+// 165 / 155.
+//
+// Grids with more workgroups than a reduction has partials (some 3.4 M nodes
+// per plane) gather too: that kernel's blocks take longer chunks instead.
 inline bool march_applies(const MarchArgs& m, int64_t bytes, int vsize, int num_cu)
 {
     const int64_t N = (int64_t)m.n0 * m.n1 * m.n2;
-    return N * vsize < ((int64_t)1 << 32) && bytes > kMallBytes && 2 * march_blocks(m) >= num_cu &&
-           march_grid(m) <= kMaxGrid;
+    if (N * vsize >= ((int64_t)1 << 32) || bytes <= kMallBytes || march_grid(m) > kMaxGrid) return false;
+    if (2 * march_blocks(m) < num_cu) return false;
+    const double steps = std::max(1.0, (double)march_blocks(m) / num_cu) * (m.zs + 1) * (num_cu / 256.0);
+    return vsize == 8 ? m.tx * m.ty >= 160 && (double)N >= 80.0 * steps * (200 + m.tx * m.ty)
+                      : (double)N >= 0.45 * 256 * kMarchThreads * steps;
 }
 
 }  // namespace rg

@@ -49,8 +49,22 @@ static void march_covers()
             }
 }
 
+// grids whose tiles leave most threads without a node, or most CUs without a
+// tile, gather (measured slower marching); the ones beside them march
+static void march_fills_the_chip()
+{
+    EXPECT(!marches(2, 2, 60000, 8) && !marches(2, 2, 60000, 4), "3 x 3 nodes per plane");
+    EXPECT(!marches(8, 8, 9000, 8) && !marches(8, 8, 9000, 4), "9 x 9 nodes per plane");
+    EXPECT(!marches(10, 10, 7000, 8) && !marches(11, 11, 5000, 8) && marches(12, 12, 4000, 8), "121, 144 and 169 nodes per plane");
+    EXPECT(!marches(64, 63, 66, 8) && marches(64, 64, 64, 8), "140 and 195 workgroups of 5 planes");
+    EXPECT(!marches(228, 228, 30, 4) && marches(228, 228, 30, 8), "130 workgroups");
+    EXPECT(!marches(30, 30, 900, 4) && marches(30, 30, 900, 8), "tiles of 8 x 31 nodes");
+    EXPECT(marches(200, 180, 40, 4) && marches(24, 24, 1500, 4) && marches(1000, 900, 3, 4), "filled tiles");
+}
+
 int main()
 {
+    march_fills_the_chip();
     march_fits_the_partials();
     march_covers();
     return bad != 0;
