@@ -326,7 +326,15 @@ struct ColourArgs {
 // colour (8 x 7 MB against 11 MB of values), 12.6 us per colour.  With a
 // contiguous range of a colour's rows per XCD (xcd_block) each pulls its part
 // of x once: 8.1 us; with the line's three neighbours by two gathers and the
-// values streamed past the caches 7.7 us.  Two lanes per row: 8.8 us.
+// values streamed past the caches (STREAM) 7.7 us.  Two lanes per row: 8.8 us.
+//
+// STREAM where the two split copies do not fit in the memory-side cache;
+// copies that do are read from there, and the second path of rows near the
+// vector's ends costs more than the gathers save.  A PCG iteration with one
+// sweep, cached / STREAM: Rectangle 60x50 51 / 57 us, 300x290 58 / 71,
+// 1000x900 (130 MB) 119 / 132, 2000x1500 (432 MB) 387 / 358; Brick 6x7x5 66 /
+// 82, 30x31x29 131 / 175, 60x61x59 152 / 187, 75x74x76 (190 MB) 175 / 222,
+// 96x95x97 (390 MB) 341 / 327, 128^3 674 / 612.
 constexpr int kSweepBlock = 64;
 
 struct SweepArgs {
@@ -345,13 +353,14 @@ struct SweepArgs {
 // FRESH: x holds rows that nothing has been written to yet; their entries are
 // zero here, and what x holds there (uninitialised memory may read as NaN) is
 // not multiplied by them.
-template <int DIM, int BS, bool FRESH>
+template <int DIM, int BS, bool FRESH, bool STREAM>
 __device__ __forceinline__ void split_product(const SweepArgs& a, const double* M, int64_t pos, int64_t row,
                                               const double* __restrict__ x, double (&acc)[BS])
 {
     constexpr int NS = StencilShape<DIM>::NS, C = StencilShape<DIM>::CENTER, B2 = BS * BS;
+    static_assert(!STREAM || BS == 1, "scalar rows");
     const int64_t reach = a.s1 + (DIM == 3 ? a.s2 : 0) + 1;
-    if (BS == 1 && row >= reach && row + reach < a.N) {
+    if (STREAM && row >= reach && row + reach < a.N) {
         // away from the vector's ends: the three neighbours of a line by one
         // 16-byte (8-byte aligned) and one 8-byte gather
 #pragma unroll
@@ -402,7 +411,7 @@ __device__ __forceinline__ void split_product(const SweepArgs& a, const double* 
 //   x_i = Dinv_i (b_i - sum_{c(k) < c(i)} A_ik x_k)
 // with Dinv the inverse main-diagonal block (Gauss-Seidel) or the inverted
 // ILU pivot (ILU).  Smoother.cpp:331-403, ILU.cpp:333-397.
-template <int DIM, int BS>
+template <int DIM, int BS, bool STREAM>
 __global__ __launch_bounds__(kSweepBlock) void k_colour_forward(SweepArgs a, int64_t p0, int64_t p1,
                                                                 const double* __restrict__ b, double* __restrict__ x)
 {
@@ -413,7 +422,7 @@ __global__ __launch_bounds__(kSweepBlock) void k_colour_forward(SweepArgs a, int
     double acc[BS];
 #pragma unroll
     for (int q = 0; q < BS; ++q) acc[q] = b[row * BS + q];
-    split_product<DIM, BS, true>(a, a.plow, pos, row, x, acc);
+    split_product<DIM, BS, true, STREAM>(a, a.plow, pos, row, x, acc);
     double out[BS];
     block_mv<BS>(a.pdinv + pos, a.ld, acc, out);
 #pragma unroll
@@ -424,7 +433,7 @@ __global__ __launch_bounds__(kSweepBlock) void k_colour_forward(SweepArgs a, int
 //   Gauss-Seidel: x_i = Dinv_i (A_ii x_i - sum_{c(k) > c(i)} A_ik x_k)
 //   ILU:          x_i = x_i - sum_{c(k) > c(i)} U_ik x_k
 // (Smoother.cpp:405-473, ILU.cpp:399-458).
-template <int DIM, int BS, bool ILU>
+template <int DIM, int BS, bool ILU, bool STREAM>
 __global__ __launch_bounds__(kSweepBlock) void k_colour_backward(SweepArgs a, int64_t p0, int64_t p1,
                                                                  double* __restrict__ x)
 {
@@ -441,7 +450,7 @@ __global__ __launch_bounds__(kSweepBlock) void k_colour_backward(SweepArgs a, in
     } else {
         block_mv<BS>(a.pdiag + pos, a.ld, xi, acc);
     }
-    split_product<DIM, BS, false>(a, a.pup, pos, row, x, acc);
+    split_product<DIM, BS, false, STREAM>(a, a.pup, pos, row, x, acc);
     if (ILU) {
 #pragma unroll
         for (int q = 0; q < BS; ++q) x[row * BS + q] = acc[q];
@@ -602,20 +611,27 @@ void colour_sweep(rg_matrix* m, const double* b, double* x, hipStream_t st, cons
 {
     const rg_colouring* c = m->colouring;
     const SweepArgs a = sweep_args(m, guard);
+    auto sweep = [&](auto D, auto B, auto S) {
+        for (int col = 0; col < c->ncolors; ++col) {
+            const int64_t p0 = c->cstart[col], p1 = c->cstart[col + 1];
+            if (p1 > p0)
+                hipLaunchKernelGGL((k_colour_forward<D.value, B.value, S.value>), dim3(sweep_blocks(p1 - p0)),
+                                   dim3(kSweepBlock), 0, st, a, p0, p1, b, x);
+        }
+        for (int col = c->ncolors - 2; col >= 0; --col) {
+            const int64_t p0 = c->cstart[col], p1 = c->cstart[col + 1];
+            if (p1 > p0)
+                hipLaunchKernelGGL((k_colour_backward<D.value, B.value, ILU, S.value>), dim3(sweep_blocks(p1 - p0)),
+                                   dim3(kSweepBlock), 0, st, a, p0, p1, x);
+        }
+    };
+    const bool stream = 2 * (int64_t)m->g.nslot * m->g.ld * (int64_t)sizeof(double) > kMallBytes;
     dispatch(m->g, false, [&](auto D, auto B, auto) {
-        if constexpr (!ILU || B.value <= 3) {
-            for (int col = 0; col < c->ncolors; ++col) {
-                const int64_t p0 = c->cstart[col], p1 = c->cstart[col + 1];
-                if (p1 > p0)
-                    hipLaunchKernelGGL((k_colour_forward<D.value, B.value>), dim3(sweep_blocks(p1 - p0)),
-                                       dim3(kSweepBlock), 0, st, a, p0, p1, b, x);
-            }
-            for (int col = c->ncolors - 2; col >= 0; --col) {
-                const int64_t p0 = c->cstart[col], p1 = c->cstart[col + 1];
-                if (p1 > p0)
-                    hipLaunchKernelGGL((k_colour_backward<D.value, B.value, ILU>), dim3(sweep_blocks(p1 - p0)),
-                                       dim3(kSweepBlock), 0, st, a, p0, p1, x);
-            }
+        if constexpr (B.value == 1) {
+            if (stream) sweep(D, B, BC<true>{});
+            else sweep(D, B, BC<false>{});
+        } else if constexpr (!ILU || B.value <= 3) {
+            sweep(D, B, BC<false>{});
         }
     });
     RG_HIP(hipGetLastError());

@@ -172,3 +172,29 @@ def test_preconditioner_errors():
         op1.solve(rhs1, _options("GAUSS_SEIDEL", method=R.SolverOptions.PCG_MIXED))
     with pytest.raises(ValueError):
         R.SolverOptions().setPreconditioner(28)   # AMG is not provided
+
+
+# split copies beyond the memory-side cache (256 MB): the substitutions stream
+# their values and gather a line's neighbours at once, but for rows near the
+# vector's ends; the first grids past that size, with odd sides
+@pytest.mark.parametrize("prec", ["GAUSS_SEIDEL", "ILU0"])
+@pytest.mark.parametrize("dim,ne", [(2, (1377, 1370)), (3, (87, 84, 86))])
+def test_streamed_substitutions_match_the_oracle(prec, dim, ne):
+    rng = np.random.default_rng(dim)
+    dom, length = grid(dim, ne)
+    E = dom.getNumElements()
+    c = {"A": np.exp(rng.standard_normal(E))[:, None, None] * np.eye(dim)[None], "D": rng.uniform(0.1, 1.0, E)}
+    op, _ = gpu_assemble(dom, 1, **c)
+    assert 2 * 3 ** dim * op.size * 8 > 1 << 28
+    ptr, idx, oval, _ = O.assemble(dim, ne, length, **c)
+    b = rng.standard_normal(op.size)
+    z = op.solvePreconditioner(to_dev(b), _options(prec)).cpu().numpy()
+    O.balance(1, ptr, idx, oval)
+    col, nc = O.coloring(ptr, idx)
+    if prec == "GAUSS_SEIDEL":
+        ref = O.gs_apply(1, ptr, idx, oval, O.inv_main(1, ptr, idx, oval), col, nc, 1, b)
+    else:
+        F, rc = O.ilu0_factor(1, ptr, idx, oval, col, nc)
+        assert rc == 0
+        ref = O.ilu0_solve(1, ptr, idx, F, col, nc, b)
+    assert np.allclose(z, ref, rtol=0, atol=1e-12 * np.abs(ref).max())
