@@ -147,7 +147,6 @@ struct AsmArgs {
     int64_t n0, n1, n2;     // nodes per axis
     int ne0, ne1, ne2;      // elements per axis
     double h0, h1, h2;
-    int reduced;
 };
 
 __device__ __forceinline__ const double* coef_pt(const CoefDev& c, int64_t e, int q, int dps)
@@ -176,15 +175,17 @@ __host__ __device__ constexpr int asm_nodes_per_wave()
 // the one-point rule of assemblePDE*Reduced (:2891-3270).  Each matrix entry
 // and rhs entry is written by exactly one thread: no atomics.
 //
-// Coefficients with one point per element (GAUSS = false) are integrated in
-// closed form (the 2-point rule is exact for these products): along an axis
+// Coefficients with one point per element (k_assemble_const) are integrated
+// in closed form (the 2-point rule is exact for these products): along an axis
 // int N N = 1/3 or 1/6 for equal / different local coordinates, int N' N =
 // +-1/2, int N' N' = +-1 in units of h, so an entry takes one multiply-add
-// per coefficient component instead of one Gauss sum.  Coefficients on
-// quadrature points and the one-point rule (GAUSS = true) take the Gauss sum,
-// the point loop outermost so that the shape functions of a point serve all
-// elements.  Both in one kernel took 256 registers (one wave per SIMD); a PDE
-// with both kinds runs a launch of each.
+// per coefficient component instead of one Gauss sum.  The one-point rule
+// differs in int N N = 1/4 only (ONE): as a Gauss sum its single point paid
+// the staging for nothing, A, D, X, Y on Brick 70x60x50 113 us, closed form
+// 66 us (the whole call).  Coefficients on quadrature points (k_assemble_gauss) take the
+// Gauss sum, the point loop outermost so that the shape functions of a point
+// serve all elements.  Both in one kernel took 256 registers (one wave per
+// SIMD); a PDE with both kinds runs a launch of each.
 //
 // Bound: the coefficient reads.  A data point of a system is NB^2 DIM^2 (A)
 // contiguous doubles of which thread (k, m) needs every NB-th, so the lanes
@@ -250,7 +251,7 @@ __device__ __forceinline__ void asm_store(const AsmNode<DIM, NB>& nd, const doub
     }
 }
 
-template <int DIM, int NB, bool SYM>
+template <int DIM, int NB, bool SYM, bool ONE>
 __global__ __launch_bounds__(kBlock) void k_assemble_const(AsmArgs a, double* __restrict__ val, int64_t ld,
                                                            int64_t tiles_x, int64_t tiles_y, bool zero,
                                                            double* __restrict__ rhs)
@@ -315,7 +316,7 @@ __global__ __launch_bounds__(kBlock) void k_assemble_const(AsmArgs a, double* __
                     const int ab = 1 - ((t >> p) & 1), bb = (b >> p) & 1;
                     sa[p] = ab ? 1.0 : -1.0;
                     sb[p] = bb ? 1.0 : -1.0;
-                    mass[p] = ab == bb ? 1.0 / 3.0 : 1.0 / 6.0;
+                    mass[p] = ONE ? 0.25 : ab == bb ? 1.0 / 3.0 : 1.0 / 6.0;
                 }
                 double full = 1.0, r = acc[s];
 #pragma unroll
@@ -460,8 +461,7 @@ __global__ __launch_bounds__(kBlock) void k_assemble_gauss(AsmArgs a, double* __
 #pragma unroll
     for (int s = 0; s < NS; ++s) acc[s] = 0.0;
     double f = 0.0;
-    const int nq = a.reduced ? 1 : NNODE;
-    const double w = vol / nq;
+    const double w = vol / NNODE;
     const double g0 = 0.5 - 0.5 / 1.73205080756887719318, g1 = 0.5 + 0.5 / 1.73205080756887719318;
     // element t of the node in LDS
     const int e0 = (min(lane / (NB * NB), Blk::EX - 2) +
@@ -472,7 +472,7 @@ __global__ __launch_bounds__(kBlock) void k_assemble_gauss(AsmArgs a, double* __
     constexpr bool AHEAD = !AGROUP && NB > 1;
     if (AHEAD) fetch_point(0);
 #pragma unroll 1
-    for (int q = 0; q < nq; ++q) {
+    for (int q = 0; q < NNODE; ++q) {
         __syncthreads();
         if (!AHEAD) fetch_point(q);
         if constexpr (AGROUP) {
@@ -485,11 +485,11 @@ __global__ __launch_bounds__(kBlock) void k_assemble_gauss(AsmArgs a, double* __
             store(a.Y, fY, IC<Blk::dpsY>{}, oY);
         }
         __syncthreads();
-        if (AHEAD && q + 1 < nq) fetch_point(q + 1);
+        if (AHEAD && q + 1 < NNODE) fetch_point(q + 1);
         double phi[DIM][2];   // 1-D shape functions at the point
 #pragma unroll
         for (int p = 0; p < DIM; ++p) {
-            phi[p][1] = a.reduced ? 0.5 : (((q >> p) & 1) ? g1 : g0);
+            phi[p][1] = ((q >> p) & 1) ? g1 : g0;
             phi[p][0] = 1.0 - phi[p][1];
         }
         // N[b], and |dN_b/dx_p| by the bits of b along the other axes (its
@@ -843,7 +843,6 @@ void launch_assemble(rg_matrix* m, const rg_pde_coefs& c, int reduced, double* r
     a.n0 = g.nn[0]; a.n1 = g.nn[1]; a.n2 = g.nn[2];
     a.ne0 = g.ne[0]; a.ne1 = g.ne[1]; a.ne2 = g.ne[2];
     a.h0 = g.h[0]; a.h1 = g.h[1]; a.h2 = g.h[2];
-    a.reduced = reduced;
     const bool iso_const = g.bs == 1 && !reduced && c.A.mode == RG_COEF_ELEMENT && c.A.isotropic && c.A.data &&
                            !c.B.mode && !c.C.mode && !c.D.mode && !c.X.mode &&
                            (c.Y.mode == RG_COEF_EMPTY || c.Y.mode == RG_COEF_ELEMENT);
@@ -894,7 +893,7 @@ void launch_assemble(rg_matrix* m, const rg_pde_coefs& c, int reduced, double* r
         bool is_const = false;
         for (auto& p : both) {
             const int mode = p[0]->mode;
-            const bool cst = !reduced && mode == RG_COEF_ELEMENT;
+            const bool cst = mode == RG_COEF_ELEMENT;
             is_const = is_const || cst;
             p[cst ? 1 : 0]->mode = RG_COEF_EMPTY;
         }
@@ -907,8 +906,12 @@ void launch_assemble(rg_matrix* m, const rg_pde_coefs& c, int reduced, double* r
             const dim3 grid((unsigned)(tx * ty * tz));
             bool zero = m->val_zero;
             if (is_const) {
-                hipLaunchKernelGGL((k_assemble_const<D.value, B.value, S.value>), grid, dim3(kBlock), 0, m->ctx->stream,
-                                   ac, m->val, g.ld, tx, ty, zero, rhs);
+                auto go = [&](auto One) {
+                    hipLaunchKernelGGL((k_assemble_const<D.value, B.value, S.value, One.value>), grid, dim3(kBlock), 0,
+                                       m->ctx->stream, ac, m->val, g.ld, tx, ty, zero, rhs);
+                };
+                if (reduced) go(BC<true>{});
+                else go(BC<false>{});
                 if (ac.A.mode || ac.B.mode || ac.C.mode || ac.D.mode) zero = false;
             }
             if (ag.A.mode) {

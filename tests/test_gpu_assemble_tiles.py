@@ -1,7 +1,7 @@
 """The gather assembly at the edges of its tiles (64 / n^2 nodes per wave along
 x, two node lines per block along y and z, four along y in 2-D) against the
-oracle: coefficients per element (closed-form integrals), on quadrature points
-(Gauss sum) and mixed, full and symmetric storage, written into zeroed values
+oracle: coefficients per element (closed-form integrals, of the 2-point and the
+one-point rule), on quadrature points (Gauss sum) and mixed, full and symmetric storage, written into zeroed values
 and added to present ones.  Bar: |d a_ij| <= 1e-13 max_j |a_ij|, as for every
 assembly."""
 import numpy as np
@@ -36,6 +36,21 @@ def test_tile_edges(n, dim, ne, expanded):
     op, rhs = gpu_assemble(dom, n, **c)
     ptr, _, val = op.exportCSR()
     _, _, oval, orhs = O.assemble(dim, ne, length, n=n, expanded=expanded, **c)
+    ok, worst = entrywise_ok(n, ptr, val, oval)
+    assert ok, worst
+    assert np.max(np.abs(rhs.cpu().numpy() - orhs)) <= 1e-13 * np.abs(orhs).max()
+
+
+@pytest.mark.parametrize("n,dim,ne", SHAPES)
+def test_one_point_rule(n, dim, ne):
+    rng = np.random.default_rng(31 * n + dim + ne[0])
+    length = tuple(0.7 + 0.3 * d for d in range(dim))
+    dom, _ = grid(dim, ne, length)
+    E = dom.getNumElements()
+    c = {k: _tensor(rng, n, dim, (E,), k) for k in "ABCDXY"}
+    op, rhs = gpu_assemble(dom, n, reduced=True, **c)
+    ptr, _, val = op.exportCSR()
+    _, _, oval, orhs = O.assemble(dim, ne, length, n=n, reduced=True, **c)
     ok, worst = entrywise_ok(n, ptr, val, oval)
     assert ok, worst
     assert np.max(np.abs(rhs.cpu().numpy() - orhs)) <= 1e-13 * np.abs(orhs).max()
