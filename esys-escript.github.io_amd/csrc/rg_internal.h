@@ -159,6 +159,7 @@ struct rg_matrix {
     bool have_prec = false;
     bool unit_jacobi = false;      // the Jacobi inverse is 1 to rounding in every row
     bool val_zero = true;          // every stored value is known to be 0 (assembly may write instead of add)
+    rg::AsmTile asm_tile[2];       // assembly: closed form, staged sums (wx 0: not chosen yet)
     rg_solver_work* work = nullptr;
     int multi_shape = 0;           // SpMM tile shape + 1 of the many-RHS solver (0: autotune)
     rg_lpc* lpc = nullptr;         // learned preconditioner (borrowed)

@@ -196,26 +196,40 @@ __host__ __device__ constexpr int asm_nodes_per_wave()
 // lanes along x, each load touched 64 lines: Brick 48x47x49, 3 equations,
 // A per element and the rest on quadrature points 10.48 ms -> 0.17 + 0.77 ms (bytes alone 0.24 ms);
 // Brick 96^3 elasticity (A per element, symmetric storage) 37.6 -> 0.92 ms (bytes alone 0.30 ms).
-template <int DIM, int NB>
+//
+// The block's nodes are those of an AsmTile: the wide one (64 / NB^2 x 2 x 2),
+// whose sides the compiler knows, or the one given (TILE, asm_tile).
+template <int DIM, int NB, bool TILE>
 struct AsmNode {
     int k, m;            // equation and component of the thread
     int64_t x, y, z, i;  // its node
     bool valid;
     int64_t e0;          // element at (x - 1, y - 1, z - 1)
     unsigned in;         // bit t: element t = (ex, ey, ez) at node index - 1 + t is in the grid
-    __device__ __forceinline__ AsmNode(const AsmArgs& a, int64_t tiles_x, int64_t tiles_y)
+    int corner;          // element (x - 1, y - 1, z - 1) among those of the block
+    __device__ __forceinline__ AsmNode(const AsmArgs& a, const AsmTile& t)
     {
         constexpr int PAIRS = NB * NB, NPW = asm_nodes_per_wave<NB>();
         const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
         const int km = lane % PAIRS;
         k = km % NB;
         m = km / NB;
-        const int64_t bx = blockIdx.x % tiles_x, by = (blockIdx.x / tiles_x) % tiles_y,
-                      bz = blockIdx.x / (tiles_x * tiles_y);
-        x = bx * NPW + lane / PAIRS;
-        y = (DIM == 3) ? by * 2 + (wv & 1) : by * 4 + wv;
-        z = (DIM == 3) ? bz * 2 + (wv >> 1) : 0;
-        valid = lane < PAIRS * NPW && x < a.n0 && y < a.n1 && (DIM == 2 || z < a.n2);
+        const int wx = TILE ? t.wx : NPW, wy = TILE ? t.wy : asm_wide_y(DIM), wz = TILE ? t.wz : asm_wide_z(DIM);
+        int lx = lane / PAIRS, ly = DIM == 3 ? wv & 1 : wv, lz = DIM == 3 ? wv >> 1 : 0;
+        bool in_tile = lane < PAIRS * NPW;
+        if (TILE) {
+            const int l = wv * NPW + lx;         // node of the tile, x fastest
+            in_tile = in_tile && l < wx * wy * wz;
+            lx = l % wx;
+            ly = (l / wx) % wy;
+            lz = DIM == 3 ? l / (wx * wy) : 0;
+        }
+        corner = in_tile ? lx + (wx + 1) * (ly + (wy + 1) * lz) : 0;
+        const int64_t bx = blockIdx.x % t.gx, by = (blockIdx.x / t.gx) % t.gy, bz = blockIdx.x / (t.gx * t.gy);
+        x = bx * wx + lx;
+        y = by * wy + ly;
+        z = DIM == 3 ? bz * wz + lz : 0;
+        valid = in_tile && x < a.n0 && y < a.n1 && (DIM == 2 || z < a.n2);
         i = x + a.n0 * (y + (DIM == 3 ? a.n1 * z : 0));
         e0 = (x - 1) + (int64_t)a.ne0 * ((y - 1) + (DIM == 3 ? (int64_t)a.ne1 * (z - 1) : 0));
         in = 0;
@@ -238,8 +252,8 @@ __host__ __device__ constexpr int asm_slot(int t, int b)
     return ((t & 1) + (b & 1)) + 3 * (((t >> 1) & 1) + ((b >> 1) & 1)) + (DIM == 3 ? 9 * ((t >> 2) + (b >> 2)) : 0);
 }
 
-template <int DIM, int NB, bool SYM>
-__device__ __forceinline__ void asm_store(const AsmNode<DIM, NB>& nd, const double (&acc)[StencilShape<DIM>::NS],
+template <int DIM, int NB, bool SYM, bool TILE>
+__device__ __forceinline__ void asm_store(const AsmNode<DIM, NB, TILE>& nd, const double (&acc)[StencilShape<DIM>::NS],
                                           double* __restrict__ val, int64_t ld, bool zero)
 {
     constexpr int FIRST = SYM ? StencilShape<DIM>::CENTER : 0;
@@ -251,14 +265,13 @@ __device__ __forceinline__ void asm_store(const AsmNode<DIM, NB>& nd, const doub
     }
 }
 
-template <int DIM, int NB, bool SYM, bool ONE>
-__global__ __launch_bounds__(kBlock) void k_assemble_const(AsmArgs a, double* __restrict__ val, int64_t ld,
-                                                           int64_t tiles_x, int64_t tiles_y, bool zero,
-                                                           double* __restrict__ rhs)
+template <int DIM, int NB, bool SYM, bool ONE, bool TILE>
+__global__ __launch_bounds__(kBlock) void k_assemble_const(AsmArgs a, AsmTile tile, double* __restrict__ val,
+                                                           int64_t ld, bool zero, double* __restrict__ rhs)
 {
     constexpr int NS = StencilShape<DIM>::NS;
     constexpr int NNODE = 1 << DIM;
-    const AsmNode<DIM, NB> nd(a, tiles_x, tiles_y);
+    const AsmNode<DIM, NB, TILE> nd(a, tile);
     if (!nd.valid) return;
     const int k = nd.k, m = nd.m;
     const double ih[3] = {1.0 / a.h0, 1.0 / a.h1, 1.0 / a.h2};
@@ -358,7 +371,7 @@ __global__ __launch_bounds__(kBlock) void k_assemble_const(AsmArgs a, double* __
         }
         __builtin_amdgcn_sched_barrier(0);   // the next element's loads stay behind: half the registers
     }
-    if (doS) asm_store<DIM, NB, SYM>(nd, acc, val, ld, zero);
+    if (doS) asm_store<DIM, NB, SYM, TILE>(nd, acc, val, ld, zero);
     if (doF) rhs[nd.i * NB + k] += f;
 }
 
@@ -373,19 +386,15 @@ __global__ __launch_bounds__(kBlock) void k_assemble_const(AsmArgs a, double* __
 // 13 us).  What is left is LDS reads and sums in turn with two barriers a point.
 template <int DIM, int NB>
 struct AsmBlock {
-    static constexpr int EX = asm_nodes_per_wave<NB>() + 1;   // elements of the block along each axis
-    static constexpr int EY = DIM == 3 ? 3 : 5;
-    static constexpr int EZ = DIM == 3 ? 3 : 1;
-    static constexpr int ELEMENTS = EX * EY * EZ;
+    static constexpr int ELEMENTS = asm_tile_elements(DIM, asm_nodes_per_wave<NB>());   // of the block, at most
     static constexpr int dpsA = NB * DIM * NB * DIM, dpsB = NB * DIM * NB, dpsD = NB * NB, dpsX = NB * DIM, dpsY = NB;
     // doubles per element of each group
     static constexpr int A_SIZE = dpsA, REST_SIZE = 2 * dpsB + dpsD + dpsX + dpsY;
 };
 
-template <int DIM, int NB, bool SYM, bool AGROUP>
-__global__ __launch_bounds__(kBlock) void k_assemble_gauss(AsmArgs a, double* __restrict__ val, int64_t ld,
-                                                           int64_t tiles_x, int64_t tiles_y, bool zero,
-                                                           double* __restrict__ rhs)
+template <int DIM, int NB, bool SYM, bool AGROUP, bool TILE>
+__global__ __launch_bounds__(kBlock) void k_assemble_gauss(AsmArgs a, AsmTile tile, double* __restrict__ val,
+                                                           int64_t ld, bool zero, double* __restrict__ rhs)
 {
     using Blk = AsmBlock<DIM, NB>;
     constexpr int NS = StencilShape<DIM>::NS;
@@ -393,9 +402,11 @@ __global__ __launch_bounds__(kBlock) void k_assemble_gauss(AsmArgs a, double* __
     constexpr int PER = AGROUP ? Blk::A_SIZE : Blk::REST_SIZE;
     constexpr int oB = 0, oC = Blk::dpsB, oD = 2 * Blk::dpsB, oX = oD + Blk::dpsD, oY = oX + Blk::dpsX;
     __shared__ double lds[Blk::ELEMENTS * PER];
-    const AsmNode<DIM, NB> nd(a, tiles_x, tiles_y);
+    const AsmNode<DIM, NB, TILE> nd(a, tile);
     const int k = nd.k, m = nd.m;
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int wx = TILE ? tile.wx : asm_nodes_per_wave<NB>(), wy = TILE ? tile.wy : asm_wide_y(DIM),
+              wz = TILE ? tile.wz : asm_wide_z(DIM);
+    const int ex = wx + 1, ey = wy + 1, elements = TILE ? ex * ey * (DIM == 3 ? wz + 1 : 1) : Blk::ELEMENTS;
     const double ih[3] = {1.0 / a.h0, 1.0 / a.h1, 1.0 / a.h2};
     double vol = a.h0 * a.h1;
     if (DIM == 3) vol *= a.h2;
@@ -404,12 +415,11 @@ __global__ __launch_bounds__(kBlock) void k_assemble_gauss(AsmArgs a, double* __
     // grid index of each element of the block, -1 outside the grid
     __shared__ int64_t index[Blk::ELEMENTS];
     {
-        const int64_t bx = blockIdx.x % tiles_x, by = (blockIdx.x / tiles_x) % tiles_y,
-                      bz = blockIdx.x / (tiles_x * tiles_y);
-        for (int el = threadIdx.x; el < Blk::ELEMENTS; el += kBlock) {
-            const int64_t k0 = bx * (Blk::EX - 1) - 1 + el % Blk::EX,
-                          k1 = by * (Blk::EY - 1) - 1 + (el / Blk::EX) % Blk::EY,
-                          k2 = DIM == 3 ? bz * (Blk::EZ - 1) - 1 + el / (Blk::EX * Blk::EY) : 0;
+        const int64_t bx = blockIdx.x % tile.gx, by = (blockIdx.x / tile.gx) % tile.gy,
+                      bz = blockIdx.x / (tile.gx * tile.gy);
+        for (int el = threadIdx.x; el < elements; el += kBlock) {
+            const int64_t k0 = bx * wx - 1 + el % ex, k1 = by * wy - 1 + (el / ex) % ey,
+                          k2 = DIM == 3 ? bz * wz - 1 + el / (ex * ey) : 0;
             const bool in = k0 >= 0 && k0 < a.ne0 && k1 >= 0 && k1 < a.ne1 && (DIM == 2 || (k2 >= 0 && k2 < a.ne2));
             index[el] = in ? k0 + (int64_t)a.ne0 * (k1 + (int64_t)a.ne1 * k2) : -1;
         }
@@ -428,7 +438,7 @@ __global__ __launch_bounds__(kBlock) void k_assemble_gauss(AsmArgs a, double* __
         for (int u = 0; u < (Blk::ELEMENTS * DPS + kBlock - 1) / kBlock; ++u) {
             const int idx = tid + u * kBlock, el = idx / DPS, o = idx % DPS;
             v[u] = 0.0;
-            if (idx < Blk::ELEMENTS * DPS && o < point) {
+            if (idx < elements * DPS && o < point) {
                 const int64_t e = index[el];
                 if (e >= 0) v[u] = p[e * c.stride + o];
             }
@@ -440,7 +450,7 @@ __global__ __launch_bounds__(kBlock) void k_assemble_gauss(AsmArgs a, double* __
 #pragma unroll
         for (int u = 0; u < (Blk::ELEMENTS * DPS + kBlock - 1) / kBlock; ++u) {
             const int idx = threadIdx.x + u * kBlock;
-            if (idx < Blk::ELEMENTS * DPS) lds[idx / DPS * PER + offset + idx % DPS] = v[u];
+            if (idx < elements * DPS) lds[idx / DPS * PER + offset + idx % DPS] = v[u];
         }
     };
     constexpr auto trips = [](int dps) { return (Blk::ELEMENTS * dps + kBlock - 1) / kBlock; };
@@ -463,9 +473,7 @@ __global__ __launch_bounds__(kBlock) void k_assemble_gauss(AsmArgs a, double* __
     double f = 0.0;
     const double w = vol / NNODE;
     const double g0 = 0.5 - 0.5 / 1.73205080756887719318, g1 = 0.5 + 0.5 / 1.73205080756887719318;
-    // element t of the node in LDS
-    const int e0 = (min(lane / (NB * NB), Blk::EX - 2) +
-                    Blk::EX * (DIM == 3 ? (wv & 1) + Blk::EY * (wv >> 1) : wv)) * PER;
+    const int e0 = nd.corner * PER;   // the node's first element in LDS
     // the next point's loads during the sums of this one: for systems other
     // than A (A's points beside its sums took more than 256 registers; a
     // single PDE's few doubles gain nothing: 94 -> 104 us)
@@ -516,7 +524,7 @@ __global__ __launch_bounds__(kBlock) void k_assemble_gauss(AsmArgs a, double* __
         };
 #pragma unroll
         for (int t = 0; t < NNODE; ++t) {
-            const double* P = lds + e0 + ((t & 1) + Blk::EX * (((t >> 1) & 1) + Blk::EY * (t >> 2))) * PER;
+            const double* P = lds + e0 + ((t & 1) + ex * (((t >> 1) & 1) + ey * (t >> 2))) * PER;
             const int la = (NNODE - 1) - t;   // the node's local index in element t
             double u[DIM], c0 = 0.0;
 #pragma unroll
@@ -570,7 +578,7 @@ __global__ __launch_bounds__(kBlock) void k_assemble_gauss(AsmArgs a, double* __
     if (doS) {
 #pragma unroll
         for (int s = 0; s < NS; ++s) acc[s] *= w;
-        asm_store<DIM, NB, SYM>(nd, acc, val, ld, zero);
+        asm_store<DIM, NB, SYM, TILE>(nd, acc, val, ld, zero);
     }
     if (doF) rhs[nd.i * NB + k] += w * f;
 }
@@ -899,29 +907,38 @@ void launch_assemble(rg_matrix* m, const rg_pde_coefs& c, int reduced, double* r
         }
         dispatch(g, m->symmetric, [&](auto D, auto B, auto S) {
             constexpr int npw = asm_nodes_per_wave<B.value>();
-            const int64_t ly = D.value == 3 ? 2 : 4;   // node lines per block along y (and 2 along z in 3-D)
-            const int64_t tx = (g.nn[0] + npw - 1) / npw, ty = (g.nn[1] + ly - 1) / ly,
-                          tz = D.value == 3 ? (g.nn[2] + 1) / 2 : 1;
-            RG_CHECK(tx * ty * tz < ((int64_t)1 << 31), RG_VALUE_ERROR, "assemble: grid too large");
-            const dim3 grid((unsigned)(tx * ty * tz));
+            // f(TILE, tile, grid) with the tile of the closed form (0) or of the staged sums (1)
+            auto with_tile = [&](int staged, auto&& f) {
+                AsmTile& t = m->asm_tile[staged];
+                if (!t.wx) t = asm_tile(D.value, g.nn, npw, staged);
+                RG_CHECK(t.gx * t.gy * t.gz < ((int64_t)1 << 31), RG_VALUE_ERROR, "assemble: grid too large");
+                const dim3 grid((unsigned)(t.gx * t.gy * t.gz));
+                if (asm_is_wide(t, D.value, npw)) f(BC<false>{}, t, grid);
+                else f(BC<true>{}, t, grid);
+            };
             bool zero = m->val_zero;
             if (is_const) {
-                auto go = [&](auto One) {
-                    hipLaunchKernelGGL((k_assemble_const<D.value, B.value, S.value, One.value>), grid, dim3(kBlock), 0,
-                                       m->ctx->stream, ac, m->val, g.ld, tx, ty, zero, rhs);
-                };
-                if (reduced) go(BC<true>{});
-                else go(BC<false>{});
+                with_tile(0, [&](auto T, const AsmTile& t, dim3 grid) {
+                    auto go = [&](auto One) {
+                        hipLaunchKernelGGL((k_assemble_const<D.value, B.value, S.value, One.value, T.value>), grid,
+                                           dim3(kBlock), 0, m->ctx->stream, ac, t, m->val, g.ld, zero, rhs);
+                    };
+                    if (reduced) go(BC<true>{});
+                    else go(BC<false>{});
+                });
                 if (ac.A.mode || ac.B.mode || ac.C.mode || ac.D.mode) zero = false;
             }
+            auto gauss = [&](auto AGroup) {
+                with_tile(1, [&](auto T, const AsmTile& t, dim3 grid) {
+                    hipLaunchKernelGGL((k_assemble_gauss<D.value, B.value, S.value, AGroup.value, T.value>), grid,
+                                       dim3(kBlock), 0, m->ctx->stream, ag, t, m->val, g.ld, zero, rhs);
+                });
+            };
             if (ag.A.mode) {
-                hipLaunchKernelGGL((k_assemble_gauss<D.value, B.value, S.value, true>), grid, dim3(kBlock), 0,
-                                   m->ctx->stream, ag, m->val, g.ld, tx, ty, zero, rhs);
+                gauss(BC<true>{});
                 zero = false;
             }
-            if (ag.B.mode || ag.C.mode || ag.D.mode || ag.X.mode || ag.Y.mode)
-                hipLaunchKernelGGL((k_assemble_gauss<D.value, B.value, S.value, false>), grid, dim3(kBlock), 0,
-                                   m->ctx->stream, ag, m->val, g.ld, tx, ty, zero, rhs);
+            if (ag.B.mode || ag.C.mode || ag.D.mode || ag.X.mode || ag.Y.mode) gauss(BC<false>{});
         });
     }
     RG_HIP(hipGetLastError());

@@ -95,4 +95,67 @@ inline bool march_applies(const MarchArgs& m, int64_t bytes, int vsize, int num_
                       : (double)N >= 0.45 * 256 * kMarchThreads * steps;
 }
 
+// ------------------------------------------------ assembly (rg_matrix.hip)
+// Nodes of a workgroup along each axis and workgroups along each axis.
+struct AsmTile {
+    int wx = 0, wy = 0, wz = 0;
+    int64_t gx = 0, gy = 0, gz = 0;
+};
+// The wide tile, known to the compiler: npw x 2 x 2 nodes (npw x 4 in 2-D) for
+// `npw` nodes per wave and four waves, whose long side reads the coefficients
+// in runs.  No tile has more elements around its nodes.
+constexpr int asm_wide_y(int dim) { return dim == 3 ? 2 : 4; }
+constexpr int asm_wide_z(int dim) { return dim == 3 ? 2 : 1; }
+constexpr int asm_tile_elements(int dim, int npw)
+{
+    return (npw + 1) * (asm_wide_y(dim) + 1) * (dim == 3 ? asm_wide_z(dim) + 1 : 1);
+}
+
+// Tile for a grid of nn nodes.  The wide one leaves most threads without a
+// node where a grid line has few: there whole lines (wx = nn[0], contiguous in
+// memory) and as many of them as fit.  The staged sums of a Brick, whose time
+// is that of the workgroups, also take the tile of the fewest workgroups where
+// the wide one needs 5/3 as many: sides just over a multiple of npw.  Otherwise
+// the wide one is the better although it has idle threads (its index arithmetic
+// is the compiler's: two equations 40 -> 60 us with the same tile given at run
+// time).  us per call, wide / as here, with D and with A, B, C, D, X, Y on
+// quadrature points: one equation on 4x40x60 elements 55 / 29 and 190 / 96,
+// 8x8000 22 / 12 and 79 / 37, 64x64x40 99 / 77 and 490 / 318; three equations
+// on 7x40x40 74 / 65 and 268 / 188; per element (A, D) 4x40x60 37 / 18.
+inline AsmTile asm_tile(int dim, const int64_t* nn, int npw, bool staged)
+{
+    const int64_t n2 = dim == 3 ? nn[2] : 1;
+    const int nodes = 4 * npw, elements = asm_tile_elements(dim, npw);
+    auto make = [&](int wx, int wy, int wz) {
+        AsmTile t;
+        t.wx = wx;
+        t.wy = wy;
+        t.wz = wz;
+        t.gx = (nn[0] + wx - 1) / wx;
+        t.gy = (nn[1] + wy - 1) / wy;
+        t.gz = (n2 + wz - 1) / wz;
+        return t;
+    };
+    auto count = [](const AsmTile& t) { return t.gx * t.gy * t.gz; };
+    const AsmTile wide = make(npw, asm_wide_y(dim), asm_wide_z(dim));
+    const bool lines = 2 * nn[0] <= npw;
+    if (!lines && (dim == 2 || !staged)) return wide;
+    AsmTile best = wide;
+    const int from = (int)std::min<int64_t>(nodes, nn[0]);
+    for (int wx = from; wx >= (lines ? from : 1); --wx)
+        for (int wy = (int)std::min<int64_t>(nodes / wx, nn[1]); wy >= 1; --wy) {
+            const int around = (wx + 1) * (wy + 1);
+            int wz = 1;
+            if (dim == 3) wz = std::min({nodes / (wx * wy), elements / around - 1, (int)std::min<int64_t>(n2, nodes)});
+            if (wz < 1 || (dim == 2 && around > elements)) continue;
+            const AsmTile t = make(wx, wy, wz);
+            if (count(t) < count(best)) best = t;
+        }
+    return 5 * count(best) < 3 * count(wide) ? best : wide;
+}
+inline bool asm_is_wide(const AsmTile& t, int dim, int npw)
+{
+    return t.wx == npw && t.wy == asm_wide_y(dim) && t.wz == asm_wide_z(dim);
+}
+
 }  // namespace rg

@@ -62,8 +62,37 @@ static void march_fills_the_chip()
     EXPECT(marches(200, 180, 40, 4) && marches(24, 24, 1500, 4) && marches(1000, 900, 3, 4), "filled tiles");
 }
 
+// assembly tiles fit a workgroup's threads and LDS and cover the grid; short
+// lines are whole, the closed form keeps the wide tile otherwise
+static void assembly_tiles()
+{
+    const int64_t sides[] = {2, 3, 4, 5, 8, 9, 17, 31, 32, 33, 49, 64, 65, 66, 71, 97, 129, 1000};
+    for (int dim : {2, 3})
+        for (int nb : {1, 2, 3, 4}) {
+            const int npw = 64 / (nb * nb);
+            for (int64_t n0 : sides)
+                for (int64_t n1 : sides)
+                    for (int64_t n2 : {2, 7, 300})
+                        for (bool staged : {false, true}) {
+                            const int64_t nn[3] = {n0, n1, n2};
+                            const rg::AsmTile t = rg::asm_tile(dim, nn, npw, staged);
+                            const int around = (t.wx + 1) * (t.wy + 1) * (dim == 3 ? t.wz + 1 : 1);
+                            EXPECT(t.wx * t.wy * t.wz <= 4 * npw && around <= rg::asm_tile_elements(dim, npw) &&
+                                       t.wx * t.gx >= n0 && t.wy * t.gy >= n1 && (dim == 2 ? t.gz == 1 : t.wz * t.gz >= n2),
+                                   "%d-D %d equations %lld x %lld x %lld", dim, nb, (long long)n0, (long long)n1, (long long)n2);
+                            EXPECT(rg::asm_is_wide(t, dim, npw) || staged || t.wx == n0, "%lld", (long long)n0);
+                        }
+        }
+    const int64_t thin[3] = {4, 4, 4001}, cube[3] = {97, 97, 97}, over[3] = {65, 65, 41};
+    EXPECT(rg::asm_tile(3, thin, 64, false).wx == 4 && rg::asm_tile(3, thin, 64, true).wx == 4, "short lines");
+    EXPECT(rg::asm_is_wide(rg::asm_tile(3, cube, 7, true), 3, 7), "97 nodes, 3 equations");
+    EXPECT(!rg::asm_is_wide(rg::asm_tile(3, over, 64, true), 3, 64) && rg::asm_is_wide(rg::asm_tile(3, over, 64, false), 3, 64),
+           "65 nodes");
+}
+
 int main()
 {
+    assembly_tiles();
     march_fills_the_chip();
     march_fits_the_partials();
     march_covers();

@@ -76,3 +76,22 @@ def test_symmetric_storage_and_second_assembly(n, dim, ne, expanded):
     op.assemble({k: R.Coefficient(to_dev(v), shape[k], E, Q, dom.device) for k, v in (("A", A), ("D", D))}, None)
     ok, worst = entrywise_ok(n, ptr, op.exportCSR()[2], 2 * oval)
     assert ok, worst
+
+
+# grids whose lines are short against a wave (whole lines per tile) and sides
+# just over a multiple of the nodes per wave (the staged sums' own tile)
+TILES = [(1, 2, (1, 40)), (1, 2, (20, 33)), (2, 2, (4, 30)), (3, 2, (1, 20)), (4, 2, (1, 9)),
+         (1, 3, (3, 2, 9)), (1, 3, (3, 70, 1)), (1, 3, (30, 3, 5)), (1, 3, (65, 5, 3)), (2, 3, (2, 5, 6)),
+         (2, 3, (16, 4, 5)), (3, 3, (2, 3, 4)), (3, 3, (7, 5, 4)), (4, 3, (1, 3, 4))]
+
+
+@pytest.mark.parametrize("n,dim,ne", TILES)
+@pytest.mark.parametrize("expanded", [(), ("B", "C", "D", "X", "Y"), ("A", "B", "C", "D", "X", "Y")])
+def test_other_tiles(n, dim, ne, expanded):
+    test_tile_edges(n, dim, ne, expanded)
+
+
+@pytest.mark.parametrize("n,dim,ne", TILES)
+def test_other_tiles_symmetric_and_one_point(n, dim, ne):
+    test_symmetric_storage_and_second_assembly(n, dim, ne, ("D",))
+    test_one_point_rule(n, dim, ne)
