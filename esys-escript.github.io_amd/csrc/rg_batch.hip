@@ -1570,6 +1570,7 @@ struct rg_batch {
     bool built_fp32 = false;
     rg::ChunkRunner run;
     rg::ResidentBatch resident;
+    int route = 0;                  // RG_ROUTE_* of the last solve
 };
 
 namespace rg {
@@ -1731,16 +1732,23 @@ int batch_solve(rg_batch* B, double* X, const double* b, const rg_options& opt, 
     // whatever the method asks of the product); a caller that gives a
     // check_interval gets the launch sequence, whose replacements and polls
     // it sets
+    B->route = 0;
     if (opt.check_interval <= 0 && B->resident.plan(B->mats)) {
         batch_prepare(B, false);
         std::vector<KrylovState> fin;
-        if (B->resident.solve(B->mats, B->offsets, B->dinv.p, b, X, B->r.p, B->p.p, B->sts.p, opt.iter_max,
-                              opt.tolerance, 16 * kResSpins, fin)) {
+        // a workgroup waits for ones that are still at an earlier system
+        const unsigned spins = B->ctx->poll_limit ? B->ctx->poll_limit : 16 * kResSpins;
+        const ResEnd end = B->resident.solve(B->mats, B->offsets, B->dinv.p, b, X, B->r.p, B->p.p, B->sts.p,
+                                             opt.iter_max, opt.tolerance, spins, fin);
+        B->resident.state = res_next(B->resident.state, end);
+        if (end == ResEnd::done) {
+            B->route = RG_ROUTE_ONE_LAUNCH;
             fill_diagnostics(fin, now_s() - t0, dg, count);
             return batch_status(dg, count, opt.accept_failed_convergence != 0);
         }
-        B->resident.state = 2;
+        B->route = RG_ROUTE_ABANDONED;
     }
+    B->route |= RG_ROUTE_LAUNCHES;
     if (B->tile_mult <= 0) batch_autotune(B, fp32, 5, nullptr);
     batch_prepare(B, fp32);
     if (B->built_mult != B->tile_mult || B->built_fp32 != fp32) build_tiles(B, B->tile_mult, fp32);
@@ -1928,6 +1936,15 @@ int rg_batch_set_tile(rg_batch* b, int tile_mult)
         RG_CHECK(b && (tile_mult == 0 || tile_mult == 1 || tile_mult == 2 || tile_mult == 4 || tile_mult == 8),
                  RG_VALUE_ERROR, "batch_set_tile: tile multiplier must be 0 (autotune), 1, 2, 4 or 8");
         b->tile_mult = tile_mult;
+        return RG_OK;
+    });
+}
+
+int rg_batch_solve_route(const rg_batch* b, int* route)
+{
+    return batch_guard([&] {
+        RG_CHECK(b && route, RG_VALUE_ERROR, "solve_route: NULL argument");
+        *route = b->route;
         return RG_OK;
     });
 }

@@ -161,6 +161,25 @@ int rg_context_set_stream(rg_context* ctx, void* stream)
     });
 }
 
+int rg_context_set_poll_limit(rg_context* ctx, uint32_t polls)
+{
+    return guarded([&] {
+        RG_CHECK(ctx != nullptr, RG_VALUE_ERROR, "context is NULL");
+        ctx->poll_limit = polls;
+        return RG_OK;
+    });
+}
+
+int rg_matrix_solve_route(const rg_matrix* m, int* route)
+{
+    return guarded([&] {
+        check_matrix(m);
+        RG_CHECK(route != nullptr, RG_VALUE_ERROR, "solve_route: NULL argument");
+        *route = m->route;
+        return RG_OK;
+    });
+}
+
 int rg_context_synchronize(rg_context* ctx)
 {
     return guarded([&] {

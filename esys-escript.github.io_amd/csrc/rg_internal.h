@@ -103,6 +103,7 @@ struct rg_context {
     int device = 0;
     hipStream_t stream = nullptr;
     int num_cu = 256;
+    unsigned poll_limit = 0;        // rg_context_set_poll_limit
     double* partials = nullptr;     // 16 * kMaxGrid doubles of per-block partial sums
     double* pinned = nullptr;       // host-pinned staging for scalars (256 doubles)
     hipEvent_t ev = nullptr;
@@ -125,7 +126,7 @@ struct rg_solver_work {
     rg::KrylovState* st = nullptr;
     int* flag = nullptr;
     void* slots = nullptr;          // partial sums of the one-launch solve (rg_resident.hip)
-    int res_state[8] = {};          // per method: 0 not looked at, 1 fits in one launch, 2 does not
+    int res_state[8] = {};          // per method, rg::ResState
     int res_tile[8][3] = {};        // its tile sides
     hipStream_t capture = nullptr;
     hipGraphExec_t graph = nullptr;
@@ -159,6 +160,7 @@ struct rg_matrix {
     bool have_prec = false;
     bool unit_jacobi = false;      // the Jacobi inverse is 1 to rounding in every row
     bool val_zero = true;          // every stored value is known to be 0 (assembly may write instead of add)
+    int route = 0;                 // RG_ROUTE_* of the last solve
     rg::AsmTile asm_tile[2];       // assembly: closed form, staged sums (wx 0: not chosen yet)
     rg_solver_work* work = nullptr;
     int multi_shape = 0;           // SpMM tile shape + 1 of the many-RHS solver (0: autotune)

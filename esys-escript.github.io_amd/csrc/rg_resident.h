@@ -12,21 +12,34 @@ namespace rg {
 // (a poll takes about a microsecond).
 constexpr unsigned kResSpins = 1u << 20;
 
+// Whether a matrix (with one method) or a batch is solved in one launch.  An
+// attempt that stopped waiting (another process or stream held the GPU) costs
+// up to a second: the next solve tries once more, then the launch sequence
+// stays.  A refused launch is not tried again.
+enum ResState { RES_UNKNOWN = 0, RES_FITS = 1, RES_OFF = 2, RES_FITS_GAVE_UP = 3 };
+inline bool res_on(int state) { return state == RES_FITS || state == RES_FITS_GAVE_UP; }
+enum class ResEnd { done, gave_up, refused };
+inline int res_next(int state, ResEnd end)
+{
+    if (end == ResEnd::done) return RES_FITS;
+    return end == ResEnd::gave_up && state == RES_FITS ? RES_FITS_GAVE_UP : RES_OFF;
+}
+
 // Tile sides of the one-launch solve of m with this method (Jacobi, one
 // sweep); false if it does not fit in the chip's registers or the method has
 // no such form.
 bool resident_fits(const rg_matrix* m, int method, int (&t)[3]);
 size_t resident_slot_bytes();
 // Runs the Krylov loop from work->r, work->xw; work->xw is the new iterate.
-// False (xw then any iterate) if the launch was refused or a workgroup gave
-// up waiting for the others.
-bool resident_solve(rg_matrix* m, int method, const int (&t)[3], int maxit, double tol, unsigned spins,
-                    KrylovState* out);
+// Not done (rows of xw then old or new) if the launch was refused or a
+// workgroup gave up waiting for the others.
+ResEnd resident_solve(rg_matrix* m, int method, const int (&t)[3], int maxit, double tol, unsigned spins,
+                      KrylovState* out);
 
 // Many independent scalar systems (full storage, one dimension, one context)
 // by the textbook Jacobi-PCG in one launch.
 struct ResidentBatch {
-    int state = 0;               // 0 not looked at, 1 every system fits, 2 not
+    int state = RES_UNKNOWN;
     int grid = 0;                // workgroups
     std::vector<int> tile;       // sides per system
     std::vector<int> tiles;      // tiles per system
@@ -40,8 +53,9 @@ struct ResidentBatch {
     ~ResidentBatch();
     bool plan(const std::vector<rg_matrix*>& mats);
     // x from x = 0; off: the systems' offsets in dinv, b, x and the two work
-    // vectors.  False if the launch was refused or a workgroup gave up.
-    bool solve(const std::vector<rg_matrix*>& mats, const std::vector<int64_t>& off, const double* dinv, const double* b,
+    // vectors.  Not done (x then in part written) if the launch was refused or
+    // a workgroup gave up.
+    ResEnd solve(const std::vector<rg_matrix*>& mats, const std::vector<int64_t>& off, const double* dinv, const double* b,
                double* x, double* pub0, double* pub1, KrylovState* st, int maxit, double tol, unsigned spins,
                std::vector<KrylovState>& out);
 };

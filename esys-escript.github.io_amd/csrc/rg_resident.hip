@@ -975,7 +975,8 @@ ResSystem res_system(const rg_matrix* m, const double* dinv, const int (&t)[3])
 
 }  // namespace
 
-bool resident_solve(rg_matrix* m, int method, const int (&t)[3], int maxit, double tol, unsigned spins, KrylovState* out)
+ResEnd resident_solve(rg_matrix* m, int method, const int (&t)[3], int maxit, double tol, unsigned spins,
+                      KrylovState* out)
 {
     const Geom& g = m->g;
     rg_solver_work* w = m->work;
@@ -1011,13 +1012,13 @@ bool resident_solve(rg_matrix* m, int method, const int (&t)[3], int maxit, doub
     });
     if (err != hipSuccess) {
         (void)hipGetLastError();
-        return false;
+        return ResEnd::refused;
     }
     KrylovState* pin = reinterpret_cast<KrylovState*>(m->ctx->pinned);
     RG_HIP(hipMemcpyAsync(pin, w->st, sizeof(KrylovState), hipMemcpyDeviceToHost, st));
     RG_HIP(hipStreamSynchronize(st));
     *out = *pin;
-    return out->done && !out->gave_up;
+    return out->done && !out->gave_up ? ResEnd::done : ResEnd::gave_up;
 }
 
 // --------------------------------------------------------------- batches
@@ -1061,8 +1062,8 @@ ResidentBatch::~ResidentBatch()
 
 bool ResidentBatch::plan(const std::vector<rg_matrix*>& mats)
 {
-    if (state) return state == 1;
-    state = 2;
+    if (state != RES_UNKNOWN) return res_on(state);
+    state = RES_OFF;
     const rg_context* ctx = mats[0]->ctx;
     const int dim = mats[0]->g.dim, blocks = std::min(kMaxTiles, ctx->num_cu);
     const int rows = kResThreads * (dim == 2 ? kBatchRows2 : kBatchRows3), cap = rows + 3 * kResThreads;
@@ -1088,11 +1089,11 @@ bool ResidentBatch::plan(const std::vector<rg_matrix*>& mats)
         tasks.push_back(system[k]);
         tasks.push_back(rank[k]);
     }
-    state = 1;
+    state = RES_FITS;
     return true;
 }
 
-bool ResidentBatch::solve(const std::vector<rg_matrix*>& mats, const std::vector<int64_t>& off, const double* dinv,
+ResEnd ResidentBatch::solve(const std::vector<rg_matrix*>& mats, const std::vector<int64_t>& off, const double* dinv,
                           const double* b, double* x, double* pub0, double* pub1, KrylovState* st, int maxit, double tol,
                           unsigned spins, std::vector<KrylovState>& out)
 {
@@ -1147,14 +1148,14 @@ bool ResidentBatch::solve(const std::vector<rg_matrix*>& mats, const std::vector
     if (err != hipSuccess) {
         (void)hipGetLastError();
         RG_HIP(hipStreamSynchronize(s));
-        return false;
+        return ResEnd::refused;
     }
     out.resize(count);
     RG_HIP(hipMemcpyAsync(out.data(), st, sizeof(KrylovState) * count, hipMemcpyDeviceToHost, s));
     RG_HIP(hipStreamSynchronize(s));
     for (const KrylovState& k : out)
-        if (!k.done || k.gave_up) return false;
-    return true;
+        if (!k.done || k.gave_up) return ResEnd::gave_up;
+    return ResEnd::done;
 }
 
 }  // namespace rg

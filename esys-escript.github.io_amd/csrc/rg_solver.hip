@@ -1084,18 +1084,25 @@ struct SolverImpl {
     Launch spmv_launch() const { return chunked_launch(m->g.N, spmv_rows_per_thread<VT>()); }
     Launch node_launch() const { return chunked_launch(m->g.N, m->g.bs == 1 ? 2 : 1); }
 
+    // Whether the PCGs' product of values of this size marches (rg_march.h).
+    bool marches(int vsize, MarchArgs& ma) const
+    {
+        const Geom& g = m->g;
+        if (g.dim != 3 || g.bs != 3 || !m->symmetric) return false;
+        ma = march_args((int)g.nn[0], (int)g.nn[1], (int)g.nn[2], m->ctx->num_cu);
+        return march_applies(ma, (int64_t)g.nstore * 9 * g.ld * vsize, vsize, m->ctx->num_cu);
+    }
+
     // v = A p with the partials of p.v; returns their number.
     template <typename VT, bool PASO>
     int spmv_dot(const PcgArgs& asp, int grid, const VT* val)
     {
         const Geom& g = m->g;
-        if (g.dim == 3 && g.bs == 3 && m->symmetric) {
-            const MarchArgs ma = march_args((int)g.nn[0], (int)g.nn[1], (int)g.nn[2], m->ctx->num_cu);
-            if (march_applies(ma, (int64_t)g.nstore * 9 * g.ld * (int64_t)sizeof(VT), sizeof(VT), m->ctx->num_cu)) {
-                const int blocks = (int)march_grid(ma);
-                hipLaunchKernelGGL((k_spmv_dot_march<3, VT>), dim3(blocks), dim3(kMarchThreads), 0, st, asp, ma, val);
-                return blocks;
-            }
+        MarchArgs ma;
+        if (marches(sizeof(VT), ma)) {
+            const int blocks = (int)march_grid(ma);
+            hipLaunchKernelGGL((k_spmv_dot_march<3, VT>), dim3(blocks), dim3(kMarchThreads), 0, st, asp, ma, val);
+            return blocks;
         }
         dispatch(g, m->symmetric, [&](auto D, auto B, auto S) {
             hipLaunchKernelGGL((k_spmv_dot<D.value, B.value, S.value, VT, PASO>), dim3(grid), dim3(kBlock), 0, st, asp,
@@ -1434,31 +1441,46 @@ struct SolverImpl {
     // (rg_resident.hip) and one Jacobi sweep; false if it is left to the
     // launch sequence.  A caller that gives a check_interval gets the launch
     // sequence, whose host polls it sets.
-    bool one_launch(int method, int sweeps, int maxit, double tol, int* status, int* iters, double* norm)
+    bool one_launch(int method, int sweeps, int maxit, double tol, bool first, int* status, int* iters, double* norm)
     {
-        if (buffered(sweeps)) return false;
-        if (w->res_state[method] == 0) w->res_state[method] = resident_fits(m, method, w->res_tile[method]) ? 1 : 2;
-        if (w->res_state[method] != 1) return false;
+        if (buffered(sweeps) || (m->route & RG_ROUTE_ABANDONED)) return false;
+        int& state = w->res_state[method];
+        if (state == RES_UNKNOWN) state = resident_fits(m, method, w->res_tile[method]) ? RES_FITS : RES_OFF;
+        if (!res_on(state)) return false;
         KrylovState out;
-        if (!resident_solve(m, method, w->res_tile[method], maxit, tol, kResSpins, &out)) {
-            // the iterate may have moved: the launch sequence starts from its residual
-            w->res_state[method] = 2;
+        const unsigned spins = m->ctx->poll_limit ? m->ctx->poll_limit : kResSpins;
+        const ResEnd end = resident_solve(m, method, w->res_tile[method], maxit, tol, spins, &out);
+        state = res_next(state, end);
+        if (end != ResEnd::done) {
+            // xw may be old in some rows and new in others: the first outer
+            // step starts again from the initial guess, a later one (both
+            // iterates are close) from what is there
+            m->route |= RG_ROUTE_ABANDONED;
+            if (first) precondition(w->bb, w->xw, sweeps, nullptr);
             RG_HIP(hipMemcpyAsync(w->r, w->bb, sizeof(double) * w->n, hipMemcpyDeviceToDevice, st));
             launch_spmv(m, -1.0, w->xw, 1.0, w->r);
             return false;
         }
+        m->route |= RG_ROUTE_ONE_LAUNCH;
         *status = out.status;
         *iters = out.num_iter;
         *norm = out.norm;
         return true;
     }
 
-    // Runs the Krylov loop from w->r, w->xw until the state reports done.
+    // Runs the Krylov loop from w->r, w->xw until the state reports done
+    // (`first`: xw is the initial guess M^-1 b).
     // Returns (status, iterations, final norm).
-    void krylov(int method, int sweeps, int maxit, double tol, int check, bool use_graph, int* status,
+    void krylov(int method, int sweeps, int maxit, double tol, int check, bool use_graph, bool first, int* status,
                 int* iters, double* norm)
     {
-        if (polls == 0 && one_launch(method, sweeps, maxit, tol, status, iters, norm)) return;
+        if (polls == 0 && one_launch(method, sweeps, maxit, tol, first, status, iters, norm)) return;
+        m->route |= RG_ROUTE_LAUNCHES;
+        if (method == RG_METHOD_PCG || method == RG_METHOD_PCG_PLAIN || method == RG_METHOD_PCG_MIXED) {
+            MarchArgs ma;
+            if (marches(method == RG_METHOD_PCG_MIXED ? 4 : 8, ma)) m->route |= RG_ROUTE_MARCH;
+            if (method != RG_METHOD_PCG_MIXED && !buffered(sweeps) && !jacobi_inverse()) m->route |= RG_ROUTE_UNIT_INVERSE;
+        }
         // the host copy and two polling slots sit below the flag words at pinned + 128
         static_assert(3 * sizeof(KrylovState) <= 128 * sizeof(double), "KrylovState outgrew the pinned buffer");
         KrylovState h;
@@ -1699,6 +1721,7 @@ int solve(rg_matrix* m, double* x, const double* b, const rg_options& opt, rg_di
     RG_CHECK(opt.criterion == RG_CRITERION_PASO || opt.criterion == RG_CRITERION_TRUE_RESIDUAL, RG_VALUE_ERROR,
              "Solver: unknown stopping criterion.");
     const bool true_res = opt.criterion == RG_CRITERION_TRUE_RESIDUAL;
+    m->route = 0;
     ensure_work(m);
     rg_solver_work* w = m->work;
     hipStream_t st = m->ctx->stream;
@@ -1783,7 +1806,7 @@ int solve(rg_matrix* m, double* x, const double* b, const rg_options& opt, rg_di
                 lastmax = normmax;
                 int ks = 0, it = 0;
                 double kn = 0;
-                S.krylov(method, std::max(1, opt.sweeps), cntIter, tol, check, use_graph, &ks, &it, &kn);
+                S.krylov(method, std::max(1, opt.sweeps), cntIter, tol, check, use_graph, totIter == 1, &ks, &it, &kn);
                 RG_HIP(hipGetLastError());
                 totIter += it;
                 if (ks == KS_CONVERGED) {

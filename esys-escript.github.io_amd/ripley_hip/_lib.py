@@ -35,6 +35,7 @@ RG_SCRATCH_BYTES = 16 << 20
 EXPORTS = [
     "rg_last_error", "rg_version",
     "rg_context_create", "rg_context_destroy", "rg_context_set_stream", "rg_context_synchronize",
+    "rg_context_set_poll_limit", "rg_matrix_solve_route", "rg_batch_solve_route",
     "rg_matrix_create", "rg_matrix_destroy", "rg_matrix_get_info", "rg_matrix_set_values",
     "rg_matrix_reset_values", "rg_matrix_add_element_blocks", "rg_matrix_assemble",
     "rg_matrix_vector", "rg_matrix_ypAx", "rg_matrix_ypAx_host",
@@ -106,6 +107,9 @@ def load():
         "rg_context_destroy": (I, [P]),
         "rg_context_set_stream": (I, [P, P]),
         "rg_context_synchronize": (I, [P]),
+        "rg_context_set_poll_limit": (I, [P, ctypes.c_uint32]),
+        "rg_matrix_solve_route": (I, [P, ctypes.POINTER(ctypes.c_int)]),
+        "rg_batch_solve_route": (I, [P, ctypes.POINTER(ctypes.c_int)]),
         "rg_matrix_create": (I, [P, I, P, P, I, I, PP]),
         "rg_matrix_destroy": (I, [P]),
         "rg_matrix_get_info": (I, [P, P, P, P, P]),

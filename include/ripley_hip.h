@@ -60,6 +60,10 @@ int rg_context_create(int device, void* stream, rg_context** out);
 int rg_context_destroy(rg_context* ctx);
 int rg_context_set_stream(rg_context* ctx, void* stream);
 int rg_context_synchronize(rg_context* ctx);
+/* Polls after which a workgroup of a one-launch solve stops waiting for the
+ * others (0: the default, about a second).  Every workgroup then ends and the
+ * launch sequence does the solve. */
+int rg_context_set_poll_limit(rg_context* ctx, uint32_t polls);
 
 /* ------------------------------------------------------------------- matrix
  * rg_matrix_create replaces RipleyDomain::newSystemMatrix ->
@@ -308,6 +312,15 @@ int rg_solve(rg_matrix* m, double* x, const double* b, const rg_options* opt,
              rg_diagnostics* diag);
 int rg_solve_host(rg_matrix* m, double* x, const double* b, const rg_options* opt,
                   rg_diagnostics* diag);
+/* Which kernels the last rg_solve of the matrix, or the last rg_batch_solve of
+ * the batch, ran: bits of RG_ROUTE_*, 0 before the first. */
+enum { RG_ROUTE_LAUNCHES = 1,      /* a sequence of launches per iteration */
+       RG_ROUTE_ONE_LAUNCH = 2,    /* the Krylov loop in one launch */
+       RG_ROUTE_ABANDONED = 4,     /* a one-launch attempt that was refused or stopped waiting */
+       RG_ROUTE_MARCH = 8,         /* z-marching product of symmetric 3 x 3 blocks */
+       RG_ROUTE_UNIT_INVERSE = 16  /* Jacobi inverse of ones left unread */ };
+int rg_matrix_solve_route(const rg_matrix* m, int* route);
+int rg_batch_solve_route(const rg_batch* b, int* route);
 
 /* ------------------------------------------------------- binary grid I/O
  * ripley's readBinaryGrid / writeBinaryGrid at one rank (host memory, no GPU
