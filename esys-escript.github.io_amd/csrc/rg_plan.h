@@ -3,7 +3,10 @@
 #pragma once
 
 #include <algorithm>
+#include <cmath>
 #include <cstdint>
+#include <utility>
+#include <vector>
 
 namespace rg {
 
@@ -156,6 +159,80 @@ inline AsmTile asm_tile(int dim, const int64_t* nn, int npw, bool staged)
 inline bool asm_is_wide(const AsmTile& t, int dim, int npw)
 {
     return t.wx == npw && t.wy == asm_wide_y(dim) && t.wz == asm_wide_z(dim);
+}
+
+// --------------------------------------- one-launch solves (rg_resident.hip)
+// Tile sides for a grid of n nodes per axis: at most `rows` nodes and
+// `cells` padded cells per tile and `tiles` tiles.  Among the shapes that
+// fit, the one with the least estimated time per iteration: a reduction over
+// G workgroups measured 1.6 / 2.3 / 2.7 / 3.2 / 3.7 / 4.0 us for G = 1 / 8 /
+// 32 / 64 / 128 / 256, the stencil about 0.4 us (3-D) or 0.15 us (2-D) per
+// 512 rows, a halo of 1024 cells 1.5 us.  With `share` the time counts
+// G^share times: 1 for systems that compete for the workgroups.
+inline bool resident_tiles(int dim, const int64_t* nn, int rows, int cells, int tiles, int (&t)[3], double share)
+{
+    const int n[3] = {(int)nn[0], (int)nn[1], dim == 3 ? (int)nn[2] : 1};
+    double best = 1e300;
+    for (int gz = 1; gz <= std::min(n[2], tiles); ++gz) {
+        const int tz = (n[2] + gz - 1) / gz;
+        if ((n[2] + tz - 1) / tz != gz) continue;
+        for (int gy = 1; gy <= std::min(n[1], tiles / gz); ++gy) {
+            const int ty = (n[1] + gy - 1) / gy;
+            if ((n[1] + ty - 1) / ty != gy) continue;
+            for (int gx = 1; gx <= std::min(n[0], tiles / (gz * gy)); ++gx) {
+                const int tx = (n[0] + gx - 1) / gx;
+                if ((n[0] + tx - 1) / tx != gx) continue;
+                const int64_t vol = (int64_t)tx * ty * tz;
+                const int64_t pad = (int64_t)(tx + 2) * (ty + 2) * (dim == 3 ? tz + 2 : 1);
+                if (vol > rows || pad > cells) continue;
+                const int G = gx * gy * gz;
+                double cost = (G > 1 ? 2.0 * (1.4 + 0.3 * std::log2((double)G)) + 1.0 + (pad - vol) / 1024.0 : 1.0) +
+                                    (dim == 3 ? 0.4 : 0.15) * (double)((vol + 511) / 512);
+                cost *= std::pow((double)G, share);
+                if (cost < best) {
+                    best = cost;
+                    t[0] = tx;
+                    t[1] = ty;
+                    t[2] = tz;
+                }
+            }
+        }
+    }
+    return best < 1e300;
+}
+
+// Which tiles of which systems each of `blocks` workgroups runs.  Systems go
+// in descending order of their expected time (iterations grow with the
+// longest side); each takes the workgroups that are free first.  A workgroup
+// waits for the others of its system, so every list is in that one order of
+// the systems: whatever is sorted or merged here must keep it.
+inline void resident_schedule(const std::vector<double>& time, const std::vector<int>& tiles, int blocks,
+                              std::vector<int>& first, std::vector<int32_t>& system, std::vector<int32_t>& rank)
+{
+    std::vector<int> order(time.size()), by_load(blocks);
+    for (size_t j = 0; j < order.size(); ++j) order[j] = (int)j;
+    std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return time[a] > time[b]; });
+    std::vector<double> load(blocks, 0.0);
+    std::vector<std::vector<std::pair<int32_t, int32_t>>> list(blocks);
+    for (int b = 0; b < blocks; ++b) by_load[b] = b;
+    for (int j : order) {
+        std::stable_sort(by_load.begin(), by_load.end(), [&](int a, int b) { return load[a] < load[b]; });
+        const double end = load[by_load[tiles[j] - 1]] + time[j];
+        for (int k = 0; k < tiles[j]; ++k) {
+            list[by_load[k]].push_back({(int32_t)j, (int32_t)k});
+            load[by_load[k]] = end;
+        }
+    }
+    first.assign(1, 0);
+    system.clear();
+    rank.clear();
+    for (int b = 0; b < blocks; ++b) {
+        for (auto& e : list[b]) {
+            system.push_back(e.first);
+            rank.push_back(e.second);
+        }
+        first.push_back((int)system.size());
+    }
 }
 
 }  // namespace rg

@@ -32,6 +32,7 @@
 #include <vector>
 
 #include "rg_device.h"
+#include "rg_plan.h"
 #include "rg_resident.h"
 #include "rg_stencil.h"
 
@@ -203,8 +204,9 @@ __device__ __forceinline__ bool reduce_all(ResShared& sh, const Gang& a, unsigne
     return !sh.bad;
 }
 
-// Rows per thread: as many as leave the stencil rows and the method's
-// vectors in 256 registers.
+// Rows per thread: as many as leave the stencil rows and the method's vectors
+// in 256 registers (k_resident<3, PCG> spills two of them and
+// k_resident_batch<3> four; a row less would cut the systems that fit by a third).
 template <int DIM, int METHOD>
 __host__ __device__ constexpr int res_rows()
 {
@@ -702,8 +704,9 @@ __global__ __launch_bounds__(kResThreads) void k_resident(ResArgs a)
 // Textbook Jacobi-PCG of many independent systems from x = 0 (unbalanced).
 // Workgroup b runs its tasks, one tile of one system each, in order; the
 // workgroups of a system form a gang.  All workgroups are resident and every
-// list is in ascending system order, so the lowest unfinished system always
-// has all its workgroups at work.  24 Rectangles n ~ U{64..400} (1.4 M rows,
+// list is in the one order of all systems that resident_schedule takes them in,
+// so the earliest unfinished system of that order always has all its
+// workgroups at work.  24 Rectangles n ~ U{64..400} (1.4 M rows,
 // 3000 iterations of the largest): 121 ms in five launches per iteration over
 // all systems -> 33 ms.
 struct ResBatchSystem {
@@ -898,45 +901,6 @@ bool by_method(int dim, int method, F&& f)
 
 }  // namespace
 
-// Tile sides for a grid of n nodes per axis: at most `rows` nodes and
-// `cells` padded cells per tile and `tiles` tiles.  Among the shapes that
-// fit, the one with the least estimated time per iteration: a reduction over
-// G workgroups measured 1.6 / 2.3 / 2.7 / 3.2 / 3.7 / 4.0 us for G = 1 / 8 /
-// 32 / 64 / 128 / 256, the stencil about 0.4 us (3-D) or 0.15 us (2-D) per
-// 512 rows, a halo of 1024 cells 1.5 us.  With `share` the time counts
-// G^share times: 1 for systems that compete for the workgroups.
-bool resident_tiles(int dim, const int64_t* nn, int rows, int cells, int tiles, int (&t)[3], double share)
-{
-    const int n[3] = {(int)nn[0], (int)nn[1], dim == 3 ? (int)nn[2] : 1};
-    double best = 1e300;
-    for (int gz = 1; gz <= std::min(n[2], tiles); ++gz) {
-        const int tz = (n[2] + gz - 1) / gz;
-        if ((n[2] + tz - 1) / tz != gz) continue;
-        for (int gy = 1; gy <= std::min(n[1], tiles / gz); ++gy) {
-            const int ty = (n[1] + gy - 1) / gy;
-            if ((n[1] + ty - 1) / ty != gy) continue;
-            for (int gx = 1; gx <= std::min(n[0], tiles / (gz * gy)); ++gx) {
-                const int tx = (n[0] + gx - 1) / gx;
-                if ((n[0] + tx - 1) / tx != gx) continue;
-                const int64_t vol = (int64_t)tx * ty * tz;
-                const int64_t pad = (int64_t)(tx + 2) * (ty + 2) * (dim == 3 ? tz + 2 : 1);
-                if (vol > rows || pad > cells) continue;
-                const int G = gx * gy * gz;
-                double cost = (G > 1 ? 2.0 * (1.4 + 0.3 * std::log2((double)G)) + 1.0 + (pad - vol) / 1024.0 : 1.0) +
-                                    (dim == 3 ? 0.4 : 0.15) * (double)((vol + 511) / 512);
-                cost *= std::pow((double)G, share);
-                if (cost < best) {
-                    best = cost;
-                    t[0] = tx;
-                    t[1] = ty;
-                    t[2] = tz;
-                }
-            }
-        }
-    }
-    return best < 1e300;
-}
-
 bool resident_fits(const rg_matrix* m, int method, int (&t)[3])
 {
     const Geom& g = m->g;
@@ -1022,38 +986,6 @@ ResEnd resident_solve(rg_matrix* m, int method, const int (&t)[3], int maxit, do
 }
 
 // --------------------------------------------------------------- batches
-
-// Which tiles of which systems each of `blocks` workgroups runs.  Systems go
-// in descending order of their expected time (iterations grow with the
-// longest side); each takes the workgroups that are free first.
-void resident_schedule(const std::vector<double>& time, const std::vector<int>& tiles, int blocks,
-                       std::vector<int>& first, std::vector<int32_t>& system, std::vector<int32_t>& rank)
-{
-    std::vector<int> order(time.size()), by_load(blocks);
-    for (size_t j = 0; j < order.size(); ++j) order[j] = (int)j;
-    std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return time[a] > time[b]; });
-    std::vector<double> load(blocks, 0.0);
-    std::vector<std::vector<std::pair<int32_t, int32_t>>> list(blocks);
-    for (int b = 0; b < blocks; ++b) by_load[b] = b;
-    for (int j : order) {
-        std::stable_sort(by_load.begin(), by_load.end(), [&](int a, int b) { return load[a] < load[b]; });
-        const double end = load[by_load[tiles[j] - 1]] + time[j];
-        for (int k = 0; k < tiles[j]; ++k) {
-            list[by_load[k]].push_back({(int32_t)j, (int32_t)k});
-            load[by_load[k]] = end;
-        }
-    }
-    first.assign(1, 0);
-    system.clear();
-    rank.clear();
-    for (int b = 0; b < blocks; ++b) {
-        for (auto& e : list[b]) {
-            system.push_back(e.first);
-            rank.push_back(e.second);
-        }
-        first.push_back((int)system.size());
-    }
-}
 
 ResidentBatch::~ResidentBatch()
 {

@@ -90,8 +90,71 @@ static void assembly_tiles()
            "65 nodes");
 }
 
+// a batch's schedule: every tile of every system once, a workgroup has at most
+// one tile of a system, and all lists are subsequences of one order of the
+// systems -- run in that order every system finds all its workgroups
+static void schedules_end()
+{
+    unsigned seed = 1;
+    auto rnd = [&](int n) { return (int)((seed = seed * 1664525u + 1013904223u) >> 8) % n; };
+    for (int round = 0; round < 300; ++round) {
+        const int blocks = 1 + rnd(256), systems = 1 + rnd(60);
+        std::vector<double> time;
+        std::vector<int> tiles, first;
+        std::vector<int32_t> system, rank;
+        for (int j = 0; j < systems; ++j) {
+            tiles.push_back(1 + rnd(rnd(3) ? std::min(blocks, 9) : blocks));
+            time.push_back(1 + rnd(rnd(2) ? 3 : 1000));
+        }
+        rg::resident_schedule(time, tiles, blocks, first, system, rank);
+        int total = 0;
+        for (int t : tiles) total += t;
+        EXPECT((int)system.size() == total && (int)first.size() == blocks + 1 && first.back() == total, "round %d", round);
+        std::vector<std::vector<char>> seen(systems);
+        for (int j = 0; j < systems; ++j) seen[j].assign(tiles[j], 0);
+        for (size_t k = 0; k < system.size(); ++k) EXPECT(!seen[system[k]][rank[k]]++, "round %d", round);
+        // workgroups advance past a system once all its tiles are at its head
+        std::vector<int> at(first.begin(), first.end() - 1);
+        int left = total;
+        for (bool moved = true; moved && left;) {
+            moved = false;
+            std::vector<int> heads(systems, 0);
+            for (int b = 0; b < blocks; ++b)
+                if (at[b] < first[b + 1]) ++heads[system[at[b]]];
+            for (int b = 0; b < blocks; ++b)
+                if (at[b] < first[b + 1] && heads[system[at[b]]] == tiles[system[at[b]]]) {
+                    ++at[b];
+                    --left;
+                    moved = true;
+                }
+        }
+        EXPECT(left == 0, "round %d: %d blocks, %d systems stuck", round, blocks, systems);
+    }
+}
+
+// one-launch tiles hold every node, within the rows and cells of a workgroup
+static void one_launch_tiles()
+{
+    const int64_t grids[][3] = {{2, 2, 1}, {3, 2501, 1}, {701, 701, 1}, {71, 70, 68}, {4, 4, 2001}, {2, 301, 301}, {65, 65, 65}};
+    for (auto& n : grids) {
+        const int dim = n[2] == 1 ? 2 : 3, rows = 512 * (dim == 2 ? 4 : 3), cells = rows + 3 * 512;
+        int t[3] = {1, 1, 1};
+        if (!rg::resident_tiles(dim, n, rows, cells, 256, t, 0.0)) continue;
+        if (dim == 2) t[2] = 1;
+        int64_t tiles = 1, vol = 1, pad = 1;
+        for (int d = 0; d < dim; ++d) {
+            tiles *= (n[d] + t[d] - 1) / t[d];
+            vol *= t[d];
+            pad *= t[d] + 2;
+        }
+        EXPECT(tiles <= 256 && vol <= rows && pad <= cells, "%lld x %lld x %lld", (long long)n[0], (long long)n[1], (long long)n[2]);
+    }
+}
+
 int main()
 {
+    schedules_end();
+    one_launch_tiles();
     assembly_tiles();
     march_fills_the_chip();
     march_fits_the_partials();
