@@ -161,9 +161,9 @@ __global__ __launch_bounds__(kBlock) void k_apply_balance(double* __restrict__ v
 // balanced diagonal and its inverse are 1 up to the three roundings of
 // a_ii d_i d_i and the division.  If every row is, the update kernels of the
 // PCGs take M^-1 r = r and leave the inverse unread (unit_jacobi): two of the
-// ten vector streams of an iteration.  Brick 128^3, symmetric storage, textbook
-// PCG: r update 12.7 -> 10.4 us, direction update 19.3 -> 17.2 us, solve 171
-// -> 163 ms.
+// twelve vector streams of an iteration.  Brick 128^3, symmetric storage, textbook
+// PCG: r update 12.7 -> 10.4 us, direction update 19.3 -> 17.2 us of some 90 us
+// per iteration (5 %; whole solves spread by as much from run to run).
 constexpr double kUnitJacobi = 1e-15;
 
 // SparseMatrix::invMain (SparseMatrix.cpp:387-435) with the closed-form
