@@ -4,6 +4,7 @@ workgroups stop waiting for one another (a poll limit of one, set by the
 host): every kernel ends, and the launch sequence gives the bits it gives when
 it is asked for."""
 import ctypes
+import threading
 
 import numpy as np
 import pytest
@@ -12,7 +13,7 @@ import torch
 import oracle as O
 import ripley_hip as R
 from gpu_helpers import to_dev
-from ripley_hip import _lib
+from ripley_hip import _lib, core
 from ripley_hip import batch as RB
 from test_gpu_march import _system as elastic_system
 from test_gpu_resident import SIZES, _batch, _problem, _solve
@@ -182,3 +183,33 @@ def test_inverse_that_is_not_one_is_read():
     o.setAcceptanceConvergenceFailureOn()
     op.solve(torch.ones(op.size, dtype=torch.float64, device="cuda"), o)
     assert route(op.handle) == LAUNCHES
+
+
+def test_threads_with_their_own_contexts(monkeypatch):
+    # cooperative launches of several streams take turns on the GPU: each
+    # solve goes through in one launch, with the bits it has alone
+    jobs = []
+    for dim, ne in MANY:
+        ctx = core.Context(0)
+        monkeypatch.setattr(core, "get_context", lambda device=0, ctx=ctx: ctx)
+        op, _, _, _, b = _problem(dim, ne, True)
+        jobs.append((op, to_dev(b), torch.cuda.Stream()))
+    monkeypatch.undo()
+    alone = [op.solve(b, options("PCG")) for op, b, _ in jobs]
+    torch.cuda.synchronize()
+    got = [[] for _ in jobs]
+
+    def work(k):
+        op, b, s = jobs[k]
+        with torch.cuda.stream(s):
+            for _ in range(8):
+                got[k].append((op.solve(b, options("PCG")), route(op.handle)))
+            s.synchronize()
+
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(len(jobs))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for x, runs in zip(alone, got):
+        assert len(runs) == 8 and all(r == ONE_LAUNCH and torch.equal(y, x) for y, r in runs)
