@@ -375,7 +375,8 @@ __global__ __launch_bounds__(kBlock) void k_assemble_const(AsmArgs a, AsmTile ti
     if (doF) rhs[nd.i * NB + k] += f;
 }
 
-// The Gauss sum of a group of coefficients: A alone (AGROUP), or B, C, D, X, Y.
+// The Gauss sum of a group of coefficients: A alone (AGROUP), or B, C, D, X, Y
+// (D alone: k_assemble_points).
 // For each quadrature point the block stages its elements' points of the
 // group in LDS (a thread per double, whole runs of a data point; zeros for
 // elements outside the grid), and every node reads its 2^DIM elements from
@@ -391,6 +392,24 @@ struct AsmBlock {
     // doubles per element of each group
     static constexpr int A_SIZE = dpsA, REST_SIZE = 2 * dpsB + dpsD + dpsX + dpsY;
 };
+
+// Grid index of each element of the block, -1 outside the grid.
+template <int DIM, int NB, bool TILE>
+__device__ __forceinline__ void asm_element_table(const AsmArgs& a, const AsmTile& tile, int64_t* index)
+{
+    const int wx = TILE ? tile.wx : asm_nodes_per_wave<NB>(), wy = TILE ? tile.wy : asm_wide_y(DIM),
+              wz = TILE ? tile.wz : asm_wide_z(DIM);
+    const int ex = wx + 1, ey = wy + 1,
+              elements = TILE ? ex * ey * (DIM == 3 ? wz + 1 : 1) : AsmBlock<DIM, NB>::ELEMENTS;
+    const int64_t bx = blockIdx.x % tile.gx, by = (blockIdx.x / tile.gx) % tile.gy,
+                  bz = blockIdx.x / (tile.gx * tile.gy);
+    for (int el = threadIdx.x; el < elements; el += kBlock) {
+        const int64_t k0 = bx * wx - 1 + el % ex, k1 = by * wy - 1 + (el / ex) % ey,
+                      k2 = DIM == 3 ? bz * wz - 1 + el / (ex * ey) : 0;
+        const bool in = k0 >= 0 && k0 < a.ne0 && k1 >= 0 && k1 < a.ne1 && (DIM == 2 || (k2 >= 0 && k2 < a.ne2));
+        index[el] = in ? k0 + (int64_t)a.ne0 * (k1 + (int64_t)a.ne1 * k2) : -1;
+    }
+}
 
 template <int DIM, int NB, bool SYM, bool AGROUP, bool TILE>
 __global__ __launch_bounds__(kBlock) void k_assemble_gauss(AsmArgs a, AsmTile tile, double* __restrict__ val,
@@ -412,19 +431,9 @@ __global__ __launch_bounds__(kBlock) void k_assemble_gauss(AsmArgs a, AsmTile ti
     if (DIM == 3) vol *= a.h2;
     const bool doS = AGROUP || (a.B.mode | a.C.mode | a.D.mode) != 0;
     const bool doF = !AGROUP && rhs != nullptr && m == 0 && (a.X.mode | a.Y.mode) != 0;
-    // grid index of each element of the block, -1 outside the grid
     __shared__ int64_t index[Blk::ELEMENTS];
-    {
-        const int64_t bx = blockIdx.x % tile.gx, by = (blockIdx.x / tile.gx) % tile.gy,
-                      bz = blockIdx.x / (tile.gx * tile.gy);
-        for (int el = threadIdx.x; el < elements; el += kBlock) {
-            const int64_t k0 = bx * wx - 1 + el % ex, k1 = by * wy - 1 + (el / ex) % ey,
-                          k2 = DIM == 3 ? bz * wz - 1 + el / (ex * ey) : 0;
-            const bool in = k0 >= 0 && k0 < a.ne0 && k1 >= 0 && k1 < a.ne1 && (DIM == 2 || (k2 >= 0 && k2 < a.ne2));
-            index[el] = in ? k0 + (int64_t)a.ne0 * (k1 + (int64_t)a.ne1 * k2) : -1;
-        }
-        __syncthreads();
-    }
+    asm_element_table<DIM, NB, TILE>(a, tile, index);
+    __syncthreads();
     // the points of quadrature point q of one coefficient, DPS doubles each:
     // loaded into registers (ahead, see AHEAD), then stored
     auto fetch = [&](const CoefDev& c, auto& v, auto dps, int q) {
@@ -581,6 +590,78 @@ __global__ __launch_bounds__(kBlock) void k_assemble_gauss(AsmArgs a, AsmTile ti
         asm_store<DIM, NB, SYM, TILE>(nd, acc, val, ld, zero);
     }
     if (doF) rhs[nd.i * NB + k] += w * f;
+}
+
+// The Gauss sum of D alone on quadrature points.  Its points of all the
+// block's elements fit in the LDS at once, so they are staged in one go (whole
+// runs of memory) and summed with constant weights N_a N_b: one barrier instead
+// of two per point, which k_assemble_gauss shares among its coefficients and D
+// alone did not repay (one equation, us per call, gather kernel with a thread
+// per node / staged by points / here: 64x64x40 elements 70 / 77 / 50, 80x80x40
+// 101 / 114 / 47, 128x64x32 100 / 111 / 45; four equations 16x20x20 61 / 77 / 52).
+template <int DIM, int NB, bool SYM, bool TILE>
+__global__ __launch_bounds__(kBlock) void k_assemble_points(AsmArgs a, AsmTile tile, double* __restrict__ val, int64_t ld,
+                                                            bool zero)
+{
+    using Blk = AsmBlock<DIM, NB>;
+    constexpr int NS = StencilShape<DIM>::NS, NNODE = 1 << DIM;
+    constexpr int DPE = NNODE * Blk::dpsD, PER = DPE + 1;   // doubles per element; odd: lanes read different banks
+    __shared__ double lds[Blk::ELEMENTS * PER];
+    __shared__ int64_t index[Blk::ELEMENTS];
+    const AsmNode<DIM, NB, TILE> nd(a, tile);
+    const int ex = (TILE ? tile.wx : asm_nodes_per_wave<NB>()) + 1, ey = (TILE ? tile.wy : asm_wide_y(DIM)) + 1,
+              elements = TILE ? ex * ey * (DIM == 3 ? tile.wz + 1 : 1) : Blk::ELEMENTS;
+    asm_element_table<DIM, NB, TILE>(a, tile, index);
+    __syncthreads();
+    constexpr int TRIPS = (Blk::ELEMENTS * DPE + kBlock - 1) / kBlock;
+    double v[TRIPS];
+#pragma unroll
+    for (int u = 0; u < TRIPS; ++u) {
+        const int idx = threadIdx.x + u * kBlock;
+        v[u] = 0.0;
+        if (idx < elements * DPE) {
+            const int64_t e = index[idx / DPE];
+            if (e >= 0) v[u] = a.D.p[e * a.D.stride + idx % DPE];
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < TRIPS; ++u) {
+        const int idx = threadIdx.x + u * kBlock;
+        if (idx < elements * DPE) lds[idx / DPE * PER + idx % DPE] = v[u];
+    }
+    __syncthreads();
+    if (!nd.valid) return;
+    constexpr double near = 0.5 + 0.5 / 1.73205080756887719318, far = 0.5 - 0.5 / 1.73205080756887719318;
+    // N_b at point q: a factor per axis, by whether node and point agree on it
+    auto N = [&](int b, int q) {
+        double n = 1.0;
+#pragma unroll
+        for (int p = 0; p < DIM; ++p) n *= ((b ^ q) >> p) & 1 ? far : near;
+        return n;
+    };
+    double acc[NS];
+#pragma unroll
+    for (int s = 0; s < NS; ++s) acc[s] = 0.0;
+#pragma unroll
+    for (int t = 0; t < NNODE; ++t) {
+        const double* P = lds + (nd.corner + (t & 1) + ex * (((t >> 1) & 1) + ey * (t >> 2))) * PER + nd.k + NB * nd.m;
+#pragma unroll
+        for (int q = 0; q < NNODE; ++q) {
+            const double c = P[q * Blk::dpsD] * N((NNODE - 1) - t, q);
+#pragma unroll
+            for (int b = 0; b < NNODE; ++b) {
+                const int s = asm_slot<DIM>(t, b);
+                if (SYM && s < StencilShape<DIM>::CENTER) continue;
+                acc[s] = fma(c, N(b, q), acc[s]);
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    double w = a.h0 * a.h1 / NNODE;
+    if (DIM == 3) w *= a.h2;
+#pragma unroll
+    for (int s = 0; s < NS; ++s) acc[s] *= w;
+    asm_store<DIM, NB, SYM, TILE>(nd, acc, val, ld, zero);
 }
 
 // Element-constant isotropic A = kappa_e I (single PDE, full quadrature),
@@ -938,7 +1019,13 @@ void launch_assemble(rg_matrix* m, const rg_pde_coefs& c, int reduced, double* r
                 gauss(BC<true>{});
                 zero = false;
             }
-            if (ag.B.mode || ag.C.mode || ag.D.mode || ag.X.mode || ag.Y.mode) gauss(BC<false>{});
+            if (ag.D.mode && !(ag.B.mode || ag.C.mode || ag.X.mode || ag.Y.mode))
+                with_tile(1, [&](auto T, const AsmTile& t, dim3 grid) {
+                    hipLaunchKernelGGL((k_assemble_points<D.value, B.value, S.value, T.value>), grid, dim3(kBlock), 0,
+                                       m->ctx->stream, ag, t, m->val, g.ld, zero);
+                });
+            else if (ag.B.mode || ag.C.mode || ag.D.mode || ag.X.mode || ag.Y.mode)
+                gauss(BC<false>{});
         });
     }
     RG_HIP(hipGetLastError());

@@ -121,10 +121,10 @@ constexpr int asm_tile_elements(int dim, int npw)
 // the wide one needs 5/3 as many: sides just over a multiple of npw.  Otherwise
 // the wide one is the better although it has idle threads (its index arithmetic
 // is the compiler's: two equations 40 -> 60 us with the same tile given at run
-// time).  us per call, wide / as here, with D and with A, B, C, D, X, Y on
-// quadrature points: one equation on 4x40x60 elements 55 / 29 and 190 / 96,
-// 8x8000 22 / 12 and 79 / 37, 64x64x40 99 / 77 and 490 / 318; three equations
-// on 7x40x40 74 / 65 and 268 / 188; per element (A, D) 4x40x60 37 / 18.
+// time).  us per call, wide / as here, with C, Y and with A, B, C, D, X, Y on
+// quadrature points: one equation on 4x40x60 elements 72 / 38 and 190 / 96,
+// 8x8000 28 / 15 and 79 / 37, 64x64x40 154 / 108 and 490 / 318; three equations
+// on 7x40x40 93 / 73 and 268 / 188; per element (A, D) 4x40x60 37 / 18.
 inline AsmTile asm_tile(int dim, const int64_t* nn, int npw, bool staged)
 {
     const int64_t n2 = dim == 3 ? nn[2] : 1;

@@ -91,6 +91,20 @@ def test_other_tiles(n, dim, ne, expanded):
     test_tile_edges(n, dim, ne, expanded)
 
 
+# D alone on quadrature points: staged whole, one barrier
+@pytest.mark.parametrize("n,dim,ne", SHAPES + TILES)
+def test_mass_matrix_on_points(n, dim, ne):
+    rng = np.random.default_rng(17 * n + dim + ne[0])
+    length = tuple(0.7 + 0.3 * d for d in range(dim))
+    dom, _ = grid(dim, ne, length)
+    D = _tensor(rng, n, dim, (dom.getNumElements(), 1 << dim), "D")
+    op, _ = gpu_assemble(dom, n, D=D)
+    ptr, _, val = op.exportCSR()
+    _, _, oval, _ = O.assemble(dim, ne, length, n=n, expanded=("D",), D=D)
+    ok, worst = entrywise_ok(n, ptr, val, oval)
+    assert ok, worst
+
+
 @pytest.mark.parametrize("n,dim,ne", TILES)
 def test_other_tiles_symmetric_and_one_point(n, dim, ne):
     test_symmetric_storage_and_second_assembly(n, dim, ne, ("D",))
