@@ -137,19 +137,21 @@ template <int NV>
 __device__ __forceinline__ bool reduce_all(ResShared& sh, const Gang& a, unsigned& epoch, double (&v)[NV])
 {
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, G = a.size;
-    // This wave's surface values and emptied slots arrive before any slot is
-    // written: they are issued before the clobber and waited for behind it (the
-    // wait by itself does not name memory, and the barrier's workgroup fence
-    // lets agent-scope stores be in flight).  A clobber beside the wait, behind
-    // the sums, cost Rectangle 256^2 0.5 %.
-    asm volatile("" ::: "memory");
 #pragma unroll
     for (int k = 0; k < NV; ++k) {
         const double s = wave_total(v[k]);
         if (lane == 0) sh.red[k][w] = s;
     }
+    // A workgroup barrier with a full wait between its fence and itself: this
+    // wave's surface values and emptied slots are issued before the fence and
+    // have arrived before any slot is written (the fence alone lets agent-scope
+    // stores be in flight, and the wait by itself does not name memory).  As an
+    // asm with a memory clobber, before or behind the sums, it cost single
+    // methods 0.5 to 2 %.
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
     __builtin_amdgcn_s_waitcnt(0);
-    __syncthreads();
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
     if (w == 0) {
         double s[NV];
 #pragma unroll
